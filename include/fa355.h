@@ -148,6 +148,12 @@ size_t fa_bwd_workspace_bytes(const fa_bwd_args* args);
  * buffer, _kernels_backward.py:203): the smallest workspace fa_bwd accepts,
  * for callers that trade the dS tiles' memory for recomputing S and dP. */
 size_t fa_bwd_min_workspace_bytes(const fa_bwd_args* args);
+/* The workspace with which fa_bwd is fastest: fa_bwd_workspace_bytes plus,
+ * for problems with few (key tile, KV head) pairs, the fp32 partial dk / dv of
+ * a dK / dV kernel split over the query rows (dk / dv then sum in another,
+ * equally fixed, order).  Depends on the current device's CU count: query it
+ * with the launch's device current. */
+size_t fa_bwd_preferred_workspace_bytes(const fa_bwd_args* args);
 int fa_bwd(const fa_bwd_args* args, void* workspace, size_t workspace_bytes,
            void* stream);
 

@@ -4,7 +4,7 @@
 // (tilelang_fa_v100/_kernels_backward.py:10-85): every dQ row is built by one
 // wave over all keys its query sees and written once, so the result does not
 // depend on the order in which workgroups run (no atomics).  The key-
-// stationary kernels (bwd_main_kernel, bwd_main_mfma_kernel) compute dK / dV.
+// stationary bwd_main_mfma_kernel computes dK / dV.
 //
 // Per 32-query-row wave and BN-key tile, with the same register layout as
 // the forward's Oᵀ = Vᵀ Pᵀ (fa_fwd_d128.h), so that no score leaves the

@@ -1,12 +1,13 @@
-// Key-stationary attention backward (dK, dV) for head_dim 128 and 256 on gfx950.
+// Key-stationary attention backward (dK, dV) on gfx950.
 //
-// Same mathematics as bwd_main_kernel (fa_bwd.hip): per (key tile, query
-// tile) the products S = Q Kᵀ, dP = dO Vᵀ, dVᵀ += dOᵀ P and dKᵀ += Qᵀ dS, with
+// Per (key tile, query tile) the products S = Q Kᵀ, dP = dO Vᵀ, dVᵀ += dOᵀ P and dKᵀ += Qᵀ dS, with
 // P = exp2(S·scale·log2e − LSE·log2e) and dS = P (dP − rowdot)·scale (rounded
 // to 16 bits with the scale in, as the reference does,
 // tilelang_fa_v100/_kernels_backward.py:160); dQ comes from
 // the query-stationary bwd_dq_kernel (fa_bwd_dq.h).  Layout, for the gfx950
 // memory instructions:
+//  * D = 64: 128 keys per workgroup, 4 waves x 32 keys, three workgroups per
+//    CU; rows are 128 bytes.
 //  * D = 128: 256 keys per workgroup, 8 waves x 32 keys (two waves per SIMD),
 //    so every Q / dO tile fetched into LDS serves 256 keys.
 //  * D = 256: 128 keys per workgroup, 4 waves x 32 keys, one wave per SIMD
@@ -18,7 +19,8 @@
 //    (buffer_load_dwordx4 ... lds), double-buffered.  Qᵀ / dOᵀ operands come
 //    from ds_read_b64_tr_b16; nothing is transposed in registers.
 //  * K / Q / dO rows use the 16-byte-chunk swizzle of fa_fwd_d128.h on the
-//    low four chunk bits (within each 256-byte half of a 512-byte row).
+//    low four chunk bits (within each 256-byte half of a 512-byte row); 128-
+//    byte rows have their own (swz_row).
 #pragma once
 
 #include "fa355.h"
@@ -32,18 +34,31 @@ template <int D_>
 struct BwdShapeMfma {
   static constexpr int D = D_;
   static constexpr int NW = D == 128 ? 8 : 4;  // waves per workgroup
-  static constexpr int BKV = 32 * NW;       // keys per workgroup: 256 (D=128), 128 (D=256)
+  static constexpr int BKV = 32 * NW;       // keys per workgroup: 256 (D=128), else 128
   static constexpr int BQ = tiles::kBwdQueryRows;  // query rows per iteration
   static constexpr int ROWB = 2 * D;        // bytes per K / Q / dO row
   static constexpr int CPR = D / 8;         // 16-byte chunks per row
   static constexpr int RPB = 1024 / ROWB;   // rows per 1 KB DMA block
-  static constexpr int K_BYTES = BKV * ROWB;  // 64 KB
-  static constexpr int QT_BYTES = BQ * ROWB;  // 8 or 16 KB
+  static constexpr int K_BYTES = BKV * ROWB;  // 64 KB (D = 64: 16 KB)
+  static constexpr int QT_BYTES = BQ * ROWB;  // 4, 8 or 16 KB
   static constexpr int QT_BLOCKS = QT_BYTES / 1024;
-  static constexpr int WPE = NW / 4;          // waves per SIMD
-  static_assert(D == 128 || D == 256, "head_dim");
+  static constexpr int WPE = D == 64 ? tiles::kBwd64WavesPerSimd : NW / 4;  // waves per SIMD
+  static_assert(D == 64 || D == 128 || D == 256, "head_dim");
   static_assert(QT_BLOCKS % NW == 0 && (K_BYTES / 1024) % NW == 0, "DMA split");
 };
+
+// 16-byte chunk swizzle of row r.  128-byte rows (D = 64) pack two rows per
+// 256 bytes of banks, so the row's parity already selects a half and the
+// three chunk bits come from the next bits: a row read's 16 rows and a
+// transpose read's 4 rows x 4 chunks then touch every bank once (the
+// 256-byte form masked to three bits left rows r and r + 2 on one bank).
+template <int D>
+__device__ __forceinline__ int swz_row(int r) {
+  if constexpr (D == 64)
+    return (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
+  else
+    return swz_chunk(r);
+}
 
 // A operands (dOᵀ, Qᵀ) of one dVᵀ / dKᵀ product pair.
 struct TrOps {
@@ -53,9 +68,14 @@ struct TrOps {
 // MODE (MaskMode): full attention, causal, or a window band from the arguments.
 // DS: also store every computed 32 x 32 dS block to `ds` (tile layout of
 // fa_bwd_ds.h; causal or full attention) for bwd_dq_ds_kernel.
-template <class T, int D_, int MODE, bool DS = false>
+// SPLIT: the workgroup's query tiles (G heads x the tiles that see its keys)
+// are cut into nsplit consecutive pieces, one workgroup each; every piece
+// writes its fp32 dK / dV to `part` in accumulator order and
+// bwd_reduce_kernel adds the pieces in their order.
+template <class T, int D_, int MODE, bool DS = false, bool SPLIT = false>
 __global__ __launch_bounds__((64 * BwdShapeMfma<D_>::NW), (BwdShapeMfma<D_>::WPE))
-void bwd_main_mfma_kernel(fa_bwd_args a, const float* stats, uint16_t* ds) {
+void bwd_main_mfma_kernel(fa_bwd_args a, const float* stats, uint16_t* ds, float* part,
+                          int nsplit) {
   using S = BwdShapeMfma<D_>;
   constexpr bool CAUSAL = MODE != kMaskNone;  // some (query, key) pairs are outside the band
   constexpr int D = S::D;
@@ -77,10 +97,13 @@ void bwd_main_mfma_kernel(fa_bwd_args a, const float* stats, uint16_t* ds) {
   const int G = H / Hk;
   const int kvtiles = (Sk + S::BKV - 1) / S::BKV;
   // Rank 0 = key tile 0, which sees the most query rows when causal.
-  const TileHead th = xcd_tile_order(blockIdx.x, kvtiles, a.batch * Hk);
+  const TileHead th =
+      xcd_tile_order(blockIdx.x, SPLIT ? kvtiles * nsplit : kvtiles, a.batch * Hk);
   const int bh = th.bh;
   const int hk = bh % Hk, b = bh / Hk;
-  const int kv0 = th.rank * S::BKV;
+  const int kv_tile = SPLIT ? th.rank / nsplit : th.rank;
+  const int piece = SPLIT ? th.rank % nsplit : 0;
+  const int kv0 = kv_tile * S::BKV;
   // Visible pairs: the band of MODE; with kMaskNone every (query, key) pair
   // inside the bounds.
   const Band band = mode_band<MODE>(a);
@@ -105,7 +128,16 @@ void bwd_main_mfma_kernel(fa_bwd_args a, const float* stats, uint16_t* ds) {
                   (int64_t)(kvw + lr) * a.dk_stride[1] + hk * a.dk_stride[2];
   uint16_t* dvp = static_cast<uint16_t*>(a.dv) + b * a.dv_stride[0] +
                   (int64_t)(kvw + lr) * a.dv_stride[1] + hk * a.dv_stride[2];
-  asm volatile("" : "+v"(dkp), "+v"(dvp));
+  // SPLIT: the lane's slot of the wave's partial block instead (layout at
+  // bwd_reduce_kernel).
+  float* pp = nullptr;
+  if constexpr (SPLIT) {
+    pp = part + 64 * D * (((int64_t)piece * (a.batch * Hk) + bh) * (kvtiles * S::NW) +
+                          kv_tile * S::NW + wave) + 4 * lane;
+    asm volatile("" : "+v"(pp));
+  } else {
+    asm volatile("" : "+v"(dkp), "+v"(dvp));
+  }
 
   // ---- K tile -> LDS: 1 KB blocks of RPB rows; wave w loads the blocks of
   // its own key rows.
@@ -114,7 +146,7 @@ void bwd_main_mfma_kernel(fa_bwd_args a, const float* stats, uint16_t* ds) {
   for (int ii = 0; ii < KBPW; ++ii) {
     const int blk = KBPW * wave + ii;
     const int r = S::RPB * blk + lane / S::CPR;
-    const int c = (lane % S::CPR) ^ swz_chunk(r);
+    const int c = (lane % S::CPR) ^ swz_row<D>(r);
     const int n = min(kv0 + r, Sk - 1);
     global_lds16_opaque(kg + (int64_t)n * a.k_stride[1] + 8 * c, Ks + blk * 1024);
   }
@@ -132,7 +164,7 @@ void bwd_main_mfma_kernel(fa_bwd_args a, const float* stats, uint16_t* ds) {
   // offset is that base XOR an instruction constant (one register per
   // pattern instead of one per chunk).  Row offsets of 16-row multiples are
   // instruction immediates.
-  const int sw_lr = swz_chunk(lr);
+  const int sw_lr = swz_row<D>(lr);
   // Row read of chunk pair c (row lr, chunk 2c + lh):
   // 16((2c + lh) ^ sw) = 32(c ^ (sw >> 1)) + 16(lh ^ (sw & 1)).
   int rb = lr * S::ROWB + 16 * (lh ^ (sw_lr & 1)) + 32 * (sw_lr >> 1);
@@ -142,12 +174,13 @@ void bwd_main_mfma_kernel(fa_bwd_args a, const float* stats, uint16_t* ds) {
   auto rk_off = [&](int c) { return rbk ^ (32 * c); };
   // Transpose read of rows 16k + r (r = 4(lane/32) + (lane%16)/4, +8 for
   // hf = 1), columns 32dt + 16((lane/16)%2) + 4(lane%4) of a 256 B-row tile:
-  // 16((4dt + q) ^ swz(r)) = 64(dt ^ (r & 3)) + 16(q ^ ((r >> 2) & 3)).
+  // 16((4dt + q) ^ swz(r)) = 64(dt ^ (r & 3)) + 16(q ^ ((r >> 2) & 3)); with
+  // the swizzle of 128-byte rows, (r >> 1) & 1 in the place of r & 3.
   const int tr_r0 = 4 * (lane >> 5) + ((lane & 15) >> 2);
   const int tr_q = 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
   auto tr_base = [&](int hf) {
     const int r = tr_r0 + 8 * hf;
-    return r * S::ROWB + 64 * (r & 3) + 16 * (tr_q ^ ((r >> 2) & 3)) + 8 * (lane & 1);
+    return r * S::ROWB + 64 * (swz_row<D>(r) >> 2) + 16 * (tr_q ^ ((r >> 2) & 3)) + 8 * (lane & 1);
   };
   int tb0 = tr_base(0), tb1 = tr_base(1);
   auto toff = [&](int hf, int dt) { return (hf ? tb1 : tb0) ^ (64 * dt); };
@@ -184,7 +217,7 @@ void bwd_main_mfma_kernel(fa_bwd_args a, const float* stats, uint16_t* ds) {
 #pragma unroll
   for (int ii = 0; ii < BPW; ++ii) {
     const int r = S::RPB * (BPW * wave + ii) + lane / S::CPR;
-    const uint32_t c = (lane % S::CPR) ^ swz_chunk(r);
+    const uint32_t c = (lane % S::CPR) ^ swz_row<D>(r);
     q_loff[ii] = 2u * (r * (uint32_t)a.q_stride[1] + 8 * c);
     o_loff[ii] = 2u * (r * (uint32_t)a.do_stride[1] + 8 * c);
   }
@@ -202,7 +235,16 @@ void bwd_main_mfma_kernel(fa_bwd_args a, const float* stats, uint16_t* ds) {
                           (int64_t)(hk * G) * a.do_stride[2] +
                           (int64_t)(max(it1, 1) - 1) * S::BQ * os1;
   const float* s_top = stats + 2 * head_rows * Sq + (max(it1, 1) - 1) * S::BQ;
-  const float* s_i = s_top;
+  // The pieces' tiles: t0 .. t1 - 1 of the workgroup's ntot, starting at query
+  // head h0, query tile it1 - 1 - r0 (first = r0 == 0: a head's first tile).
+  int t0 = 0, t1 = ntot, h0 = 0, r0 = 0;
+  if constexpr (SPLIT) {
+    t0 = (int)((int64_t)ntot * piece / nsplit);
+    t1 = (int)((int64_t)ntot * (piece + 1) / nsplit);
+    h0 = nit > 0 ? t0 / nit : 0;
+    r0 = t0 - h0 * nit;
+  }
+  const float* s_i = s_top + 2 * h0 * Sq - r0 * S::BQ;
   // DS: the dS tile of the tile `step` computes next (same sweep order as
   // the issue side), stepped back by count(it) tiles per query tile.
   static_assert(!DS || MODE != kMaskBand, "dS tiles: causal or full attention");
@@ -214,6 +256,10 @@ void bwd_main_mfma_kernel(fa_bwd_args a, const float* stats, uint16_t* ds) {
                           dsl.prefix(max(it1, 1) - 1) + kvw / 32);
   }
   uint16_t* ds_c = ds_top;
+  if constexpr (DS && SPLIT) {
+    const int top = max(it1, 1) - 1;
+    ds_c += 1024 * (h0 * dsl.per_head() - (dsl.prefix(top) - dsl.prefix(max(top - r0, 0))));
+  }
   // Buffer resources of the tile to issue next, based at its first Q / dO
   // row and carried from tile to tile: stepping back one tile is a 64-bit
   // subtract of the base words, and num_records (bytes up to the end of the
@@ -223,8 +269,17 @@ void bwd_main_mfma_kernel(fa_bwd_args a, const float* stats, uint16_t* ds) {
   // took ~25 scalar instructions per tile.
   const uint32_t q_full = span_bytes(S::BQ, qs1, D), o_full = span_bytes(S::BQ, os1, D);
   const int n_first = min(Sq - (max(it1, 1) - 1) * S::BQ, S::BQ);
-  u32x4 rq = rsrc_words(q_top, span_bytes(n_first, qs1, D));
-  u32x4 ro = rsrc_words(o_top, span_bytes(n_first, os1, D));
+  u32x4 rq = rsrc_words(q_top + h0 * a.q_stride[2] - (int64_t)r0 * S::BQ * qs1,
+                        r0 == 0 ? span_bytes(n_first, qs1, D) : q_full);
+  u32x4 ro = rsrc_words(o_top + h0 * a.do_stride[2] - (int64_t)r0 * S::BQ * os1,
+                        r0 == 0 ? span_bytes(n_first, os1, D) : o_full);
+  if constexpr (SPLIT) {  // wave-uniform; the divisions above left them in VGPRs
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      rq[w] = __builtin_amdgcn_readfirstlane(rq[w]);
+      ro[w] = __builtin_amdgcn_readfirstlane(ro[w]);
+    }
+  }
   auto step_back = [](u32x4& r, uint64_t bytes, uint32_t span) {
     const uint64_t p = (((uint64_t)r[1]) << 32 | r[0]) - bytes;
     r[0] = (uint32_t)p;
@@ -406,8 +461,9 @@ void bwd_main_mfma_kernel(fa_bwd_args a, const float* stats, uint16_t* ds) {
       ds_c -= 1024 * dsl.count(it);
     }
   };
-  int ih = 0, ii = it1 - 1;  // tile to issue next
-  int ch = 0, ci = it1 - 1;  // tile to compute next
+  int ih = h0, ii = it1 - 1 - r0;  // tile to issue next
+  int ch = h0, ci = it1 - 1 - r0;  // tile to compute next
+  const int nt = t1 - t0;
   // Iteration t: one barrier (Q/dO tile t landed, buffers of tile t-1 free),
   // then the DMA of tile t+1 and tile t's products.  The loop covers two
   // tiles so that every buffer offset is an instruction immediate.  The
@@ -421,23 +477,23 @@ void bwd_main_mfma_kernel(fa_bwd_args a, const float* stats, uint16_t* ds) {
       wait_vmem();
   };
   bool stored = false;
-  if (ntot > 0) {
+  if (nt > 0) {
     issue_q(ii, OFF_Q0, OFF_ST0);
     advance_issue(ih, ii);
   }
-  for (int t = 0; t < ntot; t += 2) {
+  for (int t = 0; t < nt; t += 2) {
     wait_tile(stored);
     __syncthreads();
-    if (t + 1 < ntot) {
+    if (t + 1 < nt) {
       issue_q(ii, OFF_Q1, OFF_ST1);
       advance_issue(ih, ii);
     }
     stored = step(ci, OFF_Q0, OFF_O0, OFF_ST0);
     advance(ch, ci);
-    if (t + 1 >= ntot) break;
+    if (t + 1 >= nt) break;
     wait_tile(stored);
     __syncthreads();
-    if (t + 2 < ntot) {
+    if (t + 2 < nt) {
       issue_q(ii, OFF_Q0, OFF_ST0);
       advance_issue(ih, ii);
     }
@@ -453,6 +509,20 @@ void bwd_main_mfma_kernel(fa_bwd_args a, const float* stats, uint16_t* ds) {
     }
   }
 
+  if constexpr (SPLIT) {
+    // Whole 1 KB blocks per store, rows past Sk included (they are zero or
+    // never read back).
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        *reinterpret_cast<f32x4*>(pp + 256 * (4 * dt + g)) =
+            f32x4{dk[dt][4 * g], dk[dt][4 * g + 1], dk[dt][4 * g + 2], dk[dt][4 * g + 3]};
+        *reinterpret_cast<f32x4*>(pp + 256 * (4 * dt + g) + 32 * D) =
+            f32x4{dv[dt][4 * g], dv[dt][4 * g + 1], dv[dt][4 * g + 2], dv[dt][4 * g + 3]};
+      }
+    return;
+  }
   if (kvw + lr >= Sk) return;
 #pragma unroll
   for (int dt = 0; dt < D / 32; ++dt)
@@ -467,6 +537,45 @@ void bwd_main_mfma_kernel(fa_bwd_args a, const float* stats, uint16_t* ds) {
       st8(dkp + d, wk);
       st8(dvp + d, wv);
     }
+}
+
+// dK / dV from the pieces of a SPLIT launch.  Piece p of 32-key block kb of
+// (batch, KV head) bh is 64 D floats at ((p nbh + bh) nblk + kb) 64 D: dK, then
+// dV, each D / 8 blocks of 1 KB, block 4 dt + g holding lane l's
+// acc[dt][4g .. 4g + 3], i.e. key 32 kb + l % 32, columns 32 dt + 8 g +
+// 4 (l / 32) .. + 3 (the dK / dV kernel's accumulators as they are, so its
+// stores and the loads here move whole kilobytes).  One wave per (block,
+// tensor, dt); the pieces are added in their order.
+template <class T, int D>
+__global__ __launch_bounds__(256) void bwd_reduce_kernel(fa_bwd_args a, const float* part,
+                                                         int nsplit, int nblk) {
+  constexpr int DT = D / 32;
+  const int nbh = a.batch * a.num_heads_k;
+  const int64_t item = (int64_t)blockIdx.x * 4 + wave_id();
+  if (item >= (int64_t)nbh * nblk * 2 * DT) return;
+  const int dt = (int)(item % DT), tensor = (int)(item / DT % 2);
+  const int64_t blk = item / (2 * DT);  // bh * nblk + kb
+  const int bh = (int)(blk / nblk), kb = (int)(blk % nblk);
+  const int lane = threadIdx.x & 63;
+  const int row = 32 * kb + (lane & 31);
+  const float* src = part + 64 * D * blk + 32 * D * tensor + 1024 * dt + 4 * lane;
+  const int64_t step = 64 * D * (int64_t)nbh * nblk;
+  f32x4 acc[4];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) acc[g] = *reinterpret_cast<const f32x4*>(src + 256 * g);
+  for (int p = 1; p < nsplit; ++p) {
+    src += step;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) acc[g] += *reinterpret_cast<const f32x4*>(src + 256 * g);
+  }
+  if (row >= a.seqlen_k) return;
+  const int hk = bh % a.num_heads_k, b = bh / a.num_heads_k;
+  const int64_t* st = tensor ? a.dv_stride : a.dk_stride;
+  uint16_t* dst = static_cast<uint16_t*>(tensor ? a.dv : a.dk) + b * st[0] + row * st[1] +
+                  hk * st[2] + 32 * dt + 4 * (lane >> 5);
+#pragma unroll
+  for (int g = 0; g < 4; ++g)
+    st8(dst + 8 * g, u32x2{T::pack(acc[g][0], acc[g][1]), T::pack(acc[g][2], acc[g][3])});
 }
 
 }  // namespace fa

@@ -164,6 +164,11 @@ size_t fa_bwd_min_workspace_bytes(const fa_bwd_args* a) {
   return fa::bwd_min_workspace_bytes(*a);
 }
 
+size_t fa_bwd_preferred_workspace_bytes(const fa_bwd_args* a) {
+  if (check_bwd(a) != FA_OK) return 0;
+  return fa::bwd_preferred_workspace_bytes(*a);
+}
+
 int fa_bwd(const fa_bwd_args* a, void* ws, size_t ws_bytes, void* stream) {
   const int st = check_bwd(a);
   if (st != FA_OK) return st;

@@ -106,10 +106,32 @@ constexpr int kBwdQueryRows = 32;
 // S and dP in bwd_dq_kernel.
 constexpr size_t kBwdDsMaxBytes = size_t(4) << 30;
 
-// ---- backward main kernel, head_dim 64 (fa_bwd.hip)
-// 128 keys per workgroup, 64 query rows per iteration, 4 waves.
-constexpr int kBwd64Keys = 128;
-constexpr int kBwd64QueryRows = 64;
+// ---- backward dK / dV kernel, head_dim 64 (fa_bwd_mfma.h): 128 keys per
+// workgroup (4 waves x 32 keys), three workgroups per CU (164-168 VGPRs, no
+// spills).  Bound by the matrix cores and the VALU together (16 products
+// against ~450 cycles of element work per 32 x 32 tile) and by the LDS operand
+// reads.  Evidence (fa_bwd per call, us, same box, against the register-
+// staged kernel this replaced, which transposed Q / dO with VALU and wrote
+// both forms to LDS): [4, 2048, 16, 64] causal 237 -> 147, full 309 -> 265;
+// [2, 8192, 16, 64] causal 1250 -> 990; [16, 512, 16, 64] causal 93 -> 69.  K
+// in registers instead of LDS spills at three waves per SIMD and took 152 /
+// 272 / 1000 / 71 us at two.
+constexpr int kBwd64WavesPerSimd = 3;
+
+// ---- backward dK / dV in pieces (fa_bwd.hip bwd_pieces): at most
+// kBwdMaxPieces workgroups per (key tile, KV head), none with fewer than
+// kBwdPieceTiles 32-row query tiles (a workgroup's start and end cost about
+// three tiles, and the reduction another launch).  Evidence (fa_bwd per call,
+// us, bf16, for 1 / 2 / 3 / 4 / 6 / 8 pieces; the rule's choice in brackets):
+//   [1, 2048, 32/8, 128] causal   401 / 248 / 197 / 172 / 154 / 161  [5: 163]
+//   [2, 2000, 32/8, 128] causal   434 / 297 / 253 / 256 / 287 / 313  [3]
+//   [1, 8192, 8/2, 128] causal   1505 / 872 / 668 / 567 / 478 / 457  [6]
+//   [1, 2048, 8, 128] full        140 / 114 / 103 / 103 / 120 / 125  [3]
+//   [2, 2048, 16, 128] causal     162 / 178 / 204 / 244 / 316 / 378  [1]
+//   [1, 4096, 32/8, 64] causal    438 / 314 / 286 / 266 / 274 / 279  [4]
+//   [1, 8192, 8/2, 256] causal   1926 / 1175 / 914 / 832 / 897 / 875 [4]
+constexpr int kBwdMaxPieces = 16;
+constexpr int kBwdPieceTiles = 16;
 
 // ---- decode, head_dim 64 / 128 / 256 / 512, pages of at least 16 keys or of
 // at least one DMA instruction's 1024 / 2D rows (fa_decode_stream.h)

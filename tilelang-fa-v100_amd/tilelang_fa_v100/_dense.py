@@ -169,19 +169,22 @@ def _empty_bytes(n: int, device):
     return torch.empty(n, dtype=torch.uint8, device=device)
 
 
-def alloc_workspace(full: int, minimal: int, device):
-    """The backward's workspace tensor: the dS path's when the limit allows
-    it, falling back to the recompute path's when that allocation raises
+def alloc_workspace(full: int, minimal: int, device, preferred: int = 0):
+    """The backward's workspace tensor: `preferred` bytes (with the partials of
+    a split dK / dV kernel) or the dS path's `full`, the larger that the limit
+    allows, falling back to the recompute path's when the allocation raises
     torch.cuda.OutOfMemoryError."""
-    if full <= minimal:
-        return _empty_bytes(minimal, device)
-    n = choose_workspace(full, minimal, workspace_limit(device, full))
-    if n == minimal:
-        return _empty_bytes(minimal, device)
-    try:
-        return _empty_bytes(n, device)
-    except torch.cuda.OutOfMemoryError:
-        return _empty_bytes(minimal, device)
+    for want in (preferred, full) if preferred > full else (full,):
+        if want <= minimal:
+            break
+        n = choose_workspace(want, minimal, workspace_limit(device, want))
+        if n == minimal:
+            continue
+        try:
+            return _empty_bytes(n, device)
+        except torch.cuda.OutOfMemoryError:
+            continue
+    return _empty_bytes(minimal, device)
 
 
 def backward(q, k, v, out, dout, lse, softmax_scale: float, causal: bool,
@@ -197,12 +200,17 @@ def backward(q, k, v, out, dout, lse, softmax_scale: float, causal: bool,
     a = bwd_args(q, k, v, out, dout, lse, dq, dk, dv, softmax_scale, causal, deterministic,
                  window)
     lib = _lib.load()
-    full = lib.fa_bwd_workspace_bytes(ctypes.byref(a))
-    minimal = lib.fa_bwd_min_workspace_bytes(ctypes.byref(a))
-    if full == 0 or minimal == 0:
-        _lib.check(_lib.FA_E_INVALID, "fa_bwd_workspace_bytes")
-    ws = alloc_workspace(full, minimal, q.device)
-    nbytes = ws.numel()
-    _lib.check(_lib.call_on(q.device, lambda st: lib.fa_bwd(ctypes.byref(a), ws.data_ptr(),
-                                                            nbytes, st)), "fa_bwd")
+
+    def run(stream):
+        # The preferred size depends on the current device (its CU count), so
+        # it is queried with the launch's device current.
+        full = lib.fa_bwd_workspace_bytes(ctypes.byref(a))
+        minimal = lib.fa_bwd_min_workspace_bytes(ctypes.byref(a))
+        if full == 0 or minimal == 0:
+            _lib.check(_lib.FA_E_INVALID, "fa_bwd_workspace_bytes")
+        ws = alloc_workspace(full, minimal, q.device,
+                             lib.fa_bwd_preferred_workspace_bytes(ctypes.byref(a)))
+        return lib.fa_bwd(ctypes.byref(a), ws.data_ptr(), ws.numel(), stream)
+
+    _lib.check(_lib.call_on(q.device, run), "fa_bwd")
     return dq, dk, dv
