@@ -31,7 +31,13 @@ namespace fa {
 template <int D_>
 struct BwdDqShape {
   static constexpr int D = D_;
-  static constexpr int NW = D == 256 ? 4 : 8;  // waves (one per SIMD at D = 256)
+  // Waves.  D = 64: four, so that three workgroups share a CU (150 VGPRs):
+  // their barriers are independent and twice as many 128-row tiles fill the
+  // chip.  Against 8 waves, one workgroup per CU (fa_bwd per call, us, same
+  // box): [2, 8192, 16, 64] causal 968 -> 941, [4, 2048, 16, 64] causal 141 ->
+  // 140, full 259 -> 256, [1, 1500, 16, 64] causal 69 -> 61.  128 VGPRs for a
+  // second 8-wave workgroup spill (188 us for the second shape).
+  static constexpr int NW = D == 128 ? 8 : 4;
   static constexpr int BM = 32 * NW;           // query rows per workgroup
   static constexpr int BN = D == 256 ? 32 : 64;  // keys per tile
   static constexpr int ROWB = 2 * D;           // bytes per K / V row
@@ -39,10 +45,7 @@ struct BwdDqShape {
   static constexpr int RPB = 1024 / ROWB;      // rows per 1 KB DMA block
   static constexpr int TILEB = BN * ROWB;      // 8 KB (D = 64) or 16 KB per K or V tile
   static constexpr int BPW = TILEB / 1024 / NW;  // DMA blocks per wave and tile
-  static constexpr int WPE = NW / 4;           // waves per SIMD
-  // Chunk swizzle bits: all four for rows of 16 or more chunks (the low four
-  // bits of each 256-byte half at D = 256), three for 8-chunk rows.
-  static constexpr int SWZ_MASK = CPR >= 16 ? 15 : CPR - 1;
+  static constexpr int WPE = D == 64 ? 3 : NW / 4;  // waves per SIMD
   static_assert(BPW * NW * 1024 == TILEB, "DMA split");
 };
 
@@ -132,7 +135,7 @@ void bwd_dq_kernel(fa_bwd_args a, float* stats) {
   // chunk kc, d tile dt: rows 16kc + 4(lane/32) + (lane%16)/4 (+8 for the
   // upper half), columns 32dt + 16((lane/16)%2) + 4(lane%4).  The swizzle of
   // a row depends on the row modulo 16 only, so kc and kt are immediates.
-  auto swz = [](int r) { return swz_chunk(r) & S::SWZ_MASK; };
+  auto swz = [](int r) { return swz_row<D>(r); };
   int koff[D / 16];
 #pragma unroll
   for (int c = 0; c < D / 16; ++c) koff[c] = lr * S::ROWB + 16 * ((2 * c + lh) ^ swz(lr));

@@ -47,19 +47,6 @@ struct BwdShapeMfma {
   static_assert(QT_BLOCKS % NW == 0 && (K_BYTES / 1024) % NW == 0, "DMA split");
 };
 
-// 16-byte chunk swizzle of row r.  128-byte rows (D = 64) pack two rows per
-// 256 bytes of banks, so the row's parity already selects a half and the
-// three chunk bits come from the next bits: a row read's 16 rows and a
-// transpose read's 4 rows x 4 chunks then touch every bank once (the
-// 256-byte form masked to three bits left rows r and r + 2 on one bank).
-template <int D>
-__device__ __forceinline__ int swz_row(int r) {
-  if constexpr (D == 64)
-    return (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
-  else
-    return swz_chunk(r);
-}
-
 // A operands (dOᵀ, Qᵀ) of one dVᵀ / dKᵀ product pair.
 struct TrOps {
   u32x4 ao, aq;

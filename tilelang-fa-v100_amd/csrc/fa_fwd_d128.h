@@ -41,6 +41,19 @@ struct FwdShapeD128 {
 
 __device__ __forceinline__ int swz_chunk(int r) { return ((r & 3) << 2) | ((r >> 2) & 3); }
 
+// 16-byte chunk swizzle of row r.  128-byte rows (D = 64) pack two rows per
+// 256 bytes of banks, so the row's parity already selects a half and the
+// three chunk bits come from the next bits: a row read's 16 rows and a
+// transpose read's 4 rows x 4 chunks then touch every bank once (the
+// 256-byte form masked to three bits left rows r and r + 2 on one bank).
+template <int D>
+__device__ __forceinline__ int swz_row(int r) {
+  if constexpr (D == 64)
+    return (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
+  else
+    return swz_chunk(r);
+}
+
 typedef short s16x4 __attribute__((__vector_size__(4 * sizeof(short))));
 
 __device__ __forceinline__ u32x2 lds_read_tr(const char* p) {
