@@ -1,0 +1,41 @@
+"""GPU parity: paged tiles of at most 32 rows (keys split over the waves).
+
+A tile's row count is (new tokens x query heads per KV head) minus the rows of
+the tiles before it; 32 takes the key-split core and 33 the row-tile one, at
+the same shapes, in one batch with sequences that do the other.  Key counts
+sit at the edges of the 32-key tiles, of the 16-key halves that one page base
+serves, and of the ranges of 4 and 8 waves; caches hold NaN past every
+sequence's end.  Oracle bar as for the other paged paths (outputs atol 2e-3 /
+rtol 1e-2, LSE within 1e-3, relative L2 < 1e-2).
+"""
+import pytest
+import torch
+
+from test_gpu_paged import make_case
+from test_gpu_paged_split import run_split
+
+pytestmark = pytest.mark.gpu
+
+F16, BF16 = torch.float16, torch.bfloat16
+CASES = [
+    # (q_lens, seq_lens, Hq, Hkv, D, page, dtype, causal, wq, wk, splits); prefix = seq - q
+    ([1, 8, 9, 1, 1], [1, 31, 33, 257, 513], 16, 4, 128, 16, F16, True, -1, -1, 1),
+    ([1, 8, 9, 1, 200], [16, 255, 300, 2049, 260], 16, 4, 128, 64, BF16, True, -1, -1, 3),
+    ([4, 5, 0, 1], [1000, 1001, 40, 15], 64, 8, 128, 32, F16, False, -1, -1, 2),
+    ([1, 7, 32], [700, 333, 47], 8, 8, 128, 16, F16, True, 100, 30, 1),
+    ([1, 8, 9, 1], [1, 129, 140, 1025], 8, 2, 64, 16, F16, True, -1, -1, 1),
+    ([2, 33, 1], [100, 99, 4000], 7, 1, 64, 8, BF16, True, -1, -1, 4),   # pages of 8: no key split
+    ([1, 32, 1], [33, 77, 2000], 8, 8, 64, 64, F16, True, 50, -1, 2),
+    ([1, 4, 5, 1], [1, 127, 131, 1500], 16, 2, 256, 16, F16, True, -1, -1, 1),
+    ([1, 3, 140], [2000, 31, 170], 16, 2, 256, 32, BF16, True, -1, -1, 3),
+]
+
+
+@pytest.mark.parametrize("case", CASES,
+                         ids=[f"D{c[4]}-p{c[5]}-{str(c[6])[6:]}-s{c[10]}-{i}"
+                              for i, c in enumerate(CASES)])
+def test_few_row_tiles_match_oracle(case):
+    ql, sl, Hq, Hkv, D, page, dt, causal, wq, wk, ns = case
+    c = make_case(29, ql, sl, [s - q for q, s in zip(ql, sl)], Hq, Hkv, D, page=page, dtype=dt)
+    print(f"case {case}", flush=True)
+    run_split(c, ns, causal=causal, wq=wq, wk=wk)

@@ -125,6 +125,32 @@ __device__ __forceinline__ void run_fwd_tiles(Prob P, int row0, float scale, Nex
   }
 }
 
+// Row problem of query head bh % H of batch bh / H, its arguments read through
+// `ap` (a pointer to fa_fwd_args in any address space).
+template <int MODE, class ArgsPtr>
+__device__ __forceinline__ void dense_rows(const ArgsPtr ap, int bh, DenseRows& P) {
+  const int H = ap->num_heads;
+  const int h = bh % H;
+  const int b = bh / H;
+  const int hk = h / (H / ap->num_heads_k);
+  P.q = static_cast<const uint16_t*>(ap->q) + b * ap->q_stride[0] + h * ap->q_stride[2];
+  P.o = static_cast<uint16_t*>(ap->out) + b * ap->o_stride[0] + h * ap->o_stride[2];
+  P.lse = ap->lse ? ap->lse + ((int64_t)b * H + h) * ap->seqlen_q : nullptr;
+  P.k = static_cast<const uint16_t*>(ap->k) + b * ap->k_stride[0] + hk * ap->k_stride[2];
+  P.v = static_cast<const uint16_t*>(ap->v) + b * ap->v_stride[0] + hk * ap->v_stride[2];
+  P.qs = ap->q_stride[1];
+  P.os = ap->o_stride[1];
+  P.ks = ap->k_stride[1];
+  P.vs = ap->v_stride[1];
+  P.nrows = ap->seqlen_q;
+  P.sk = ap->seqlen_k;
+  P.off = ap->seqlen_k - ap->seqlen_q;
+  const Band band = mode_band<MODE>(*ap);
+  P.wl = band.wl;
+  P.wr = band.wr;
+  P.has_lse = ap->lse != nullptr;
+}
+
 // MODE (MaskMode): full attention, causal, or a window band from the
 // arguments.  The causal and full bands are compile-time constants.
 template <class T, int D, int MODE>
@@ -140,29 +166,9 @@ void fwd_dense_kernel(fa_fwd_args a) {
   auto setup = [qtiles, nbh](int vid, DenseRows& P, int& row0) {
     const auto* ap = kernel_args<fa_fwd_args>();
     const TileHead th = xcd_tile_order(vid, qtiles, nbh);
-    const int bh = th.bh;
-    const int H = ap->num_heads;
-    const int h = bh % H;
-    const int b = bh / H;
     // Heaviest causal tiles (largest query index) first.
     const int qt = MODE != kMaskNone ? qtiles - 1 - th.rank : th.rank;
-    const int hk = h / (H / ap->num_heads_k);
-    P.q = static_cast<const uint16_t*>(ap->q) + b * ap->q_stride[0] + h * ap->q_stride[2];
-    P.o = static_cast<uint16_t*>(ap->out) + b * ap->o_stride[0] + h * ap->o_stride[2];
-    P.lse = ap->lse ? ap->lse + ((int64_t)b * H + h) * ap->seqlen_q : nullptr;
-    P.k = static_cast<const uint16_t*>(ap->k) + b * ap->k_stride[0] + hk * ap->k_stride[2];
-    P.v = static_cast<const uint16_t*>(ap->v) + b * ap->v_stride[0] + hk * ap->v_stride[2];
-    P.qs = ap->q_stride[1];
-    P.os = ap->o_stride[1];
-    P.ks = ap->k_stride[1];
-    P.vs = ap->v_stride[1];
-    P.nrows = ap->seqlen_q;
-    P.sk = ap->seqlen_k;
-    P.off = ap->seqlen_k - ap->seqlen_q;
-    const Band band = mode_band<MODE>(*ap);
-    P.wl = band.wl;
-    P.wr = band.wr;
-    P.has_lse = ap->lse != nullptr;
+    dense_rows<MODE>(ap, th.bh, P);
     row0 = qt * C::BM;
   };
   DenseRows P;
@@ -185,6 +191,21 @@ void fwd_dense_kernel(fa_fwd_args a) {
     setup(v, Pn, rn);
     return true;
   });
+}
+
+// Keys split across the waves of a workgroup (fa_fwd_split.h), for grids too
+// small for the kernel above: one workgroup per 32 query rows of a head.
+constexpr int dense_split_waves(int D) {
+  return D == 64 ? tiles::kFwdSplitWaves64 : tiles::kFwdSplitWaves128;
+}
+template <class T, int D, int MODE>
+__global__ __launch_bounds__(64 * dense_split_waves(D)) void fwd_split_kernel(fa_fwd_args a) {
+  constexpr int NW = dense_split_waves(D);
+  __shared__ __attribute__((aligned(16))) char smem[FwdSplitShape<D, NW>::LDS];
+  const TileHead th = xcd_tile_order(blockIdx.x, (a.seqlen_q + 31) / 32, a.batch * a.num_heads);
+  DenseRows P;
+  dense_rows<MODE>(&a, th.bh, P);
+  attn_fwd_split_tile<T, D, NW>(P, 32 * th.rank, a.softmax_scale, smem);
 }
 
 struct PagedRows {
@@ -366,8 +387,9 @@ __device__ int find_sequence(const int32_t* qsl, const int32_t* prefix, int batc
 }
 
 // Row problem of KV head hk of sequence b (query tokens qs .. qs+qlen-1).
-__device__ __forceinline__ void paged_rows(const fa_paged_args& a, int hk, int b, int qs,
-                                           int qlen, PagedRows& P) {
+template <class Args>
+__device__ __forceinline__ void paged_rows(const Args& a, int hk, int b, int qs, int qlen,
+                                           PagedRows& P) {
   const int G = a.num_heads / a.num_kv_heads;
   P.G = G;
   P.nrows = qlen * G;
@@ -401,6 +423,50 @@ __device__ __forceinline__ void paged_rows(const fa_paged_args& a, int hk, int b
   P.wk = a.window_k;
 }
 
+// One row tile of a paged problem; setup(args, P) fills the problem from the
+// kernel's arguments.  A tile of at most 32 rows (a decoding sequence in a
+// prefill batch, or the last rows of a prompt) would keep one wave of the
+// row-tile cores busy, serially over the keys; its keys are split over the
+// waves instead (fa_fwd_split.h; pages of at least 16 keys, strides that fit
+// its 32-bit lane offsets).  Each branch sets up its own problem, the few-row
+// one from arguments the compiler reloads: with one problem for both, its
+// scalars stayed live across the ping-pong core and spilled in its loop (49
+// spilled SGPRs against 13, C5-size chunked prefill 0.7% slower).
+template <class T, int D, bool PP, class Prob, class Setup>
+__device__ __forceinline__ void run_paged_tile(const fa_paged_args& a, int rows, int row0,
+                                               Setup setup) {
+  using C = FwdKernelCfg<D, PP>;
+  if constexpr (D == 64 || (PP && (D == 128 || D == 256))) {
+    constexpr int NW = C::THREADS / 64;
+    constexpr int kSplitLds = FwdSplitShape<D, NW>::LDS;
+    constexpr int kLds = kSplitLds > C::LDS_BYTES ? kSplitLds : C::LDS_BYTES;
+    __shared__ __attribute__((aligned(16))) char smem[kLds];
+    constexpr int64_t kMaxSlot = 1 << 24;
+    if (rows <= 32 && (PP || (a.page_size >= 16 && a.k_stride[1] < kMaxSlot &&
+                              a.v_stride[1] < kMaxSlot))) {
+      const auto* ap = kernel_args<fa_paged_args>();
+      Prob P;
+      setup(*ap, P);
+      attn_fwd_split_tile<T, D, NW>(P, row0, ap->softmax_scale, smem);
+      return;
+    }
+    Prob P;
+    setup(a, P);
+    if constexpr (D == 128) {
+      constexpr int B = FwdShapeD128::LDS_ARRAY_BYTES;
+      attn_fwd_tile_d128<T>(P, row0, a.softmax_scale, smem, smem + B, smem + 2 * B, smem + 3 * B);
+    } else if constexpr (D == 256) {
+      attn_fwd_tile_1w<T, 256, 1>(P, row0, a.softmax_scale, smem);
+    } else {
+      attn_fwd_tile<T, D>(P, row0, a.softmax_scale, reinterpret_cast<uint16_t*>(smem));
+    }
+  } else {
+    Prob P;
+    setup(a, P);
+    run_fwd_tile<T, D, PP>(P, row0, a.softmax_scale);
+  }
+}
+
 template <class T, int D, bool PP>
 __global__ __launch_bounds__((FwdKernelCfg<D, PP>::THREADS), (FwdKernelCfg<D, PP>::WAVES_PER_EU))
 void fwd_paged_kernel(fa_paged_args a) {
@@ -419,9 +485,10 @@ void fwd_paged_kernel(fa_paged_args a) {
   const int ntiles = (int)(((int64_t)qlen * G + S::BM - 1) / S::BM);
   // Later tiles of a causal sequence see more keys: run them first.
   const int tile = ntiles - 1 - local;
-  PagedRows P;
-  paged_rows(a, hk, b, qs, qlen, P);
-  run_fwd_tile<T, D, PP>(P, tile * S::BM, a.softmax_scale);
+  const int row0 = tile * S::BM;
+  run_paged_tile<T, D, PP, PagedRows>(
+      a, qlen * G - row0, row0,
+      [=](const auto& args, PagedRows& P) { paged_rows(args, hk, b, qs, qlen, P); });
 }
 
 // Split-KV variant: workgroup (split, KV head, tile slot); the splits of a
@@ -447,17 +514,21 @@ void fwd_paged_split_kernel(fa_paged_args a, int nsplit, float* po, float* plse)
   const int qlen = a.query_start_loc[b + 1] - qs;
   const int ntiles = (int)(((int64_t)qlen * G + S::BM - 1) / S::BM);
   const int tile = ntiles - 1 - local;
-  PagedSplitRows P;
-  paged_rows(a, hk, b, qs, qlen, P);
-  const int chunk = ((P.seq_len + nsplit - 1) / nsplit + 127) / 128 * 128;
-  P.split_lo = split * chunk;
-  P.split_hi = P.split_lo + chunk;
-  const int64_t origin = ((int64_t)split * a.num_heads + (int64_t)hk * G) * a.num_tokens + qs;
-  P.po = po + origin * D;
-  P.plse = plse + origin;
-  P.p_head = a.num_tokens;
-  P.D = D;
-  run_fwd_tile<T, D, PP>(P, tile * S::BM, a.softmax_scale);
+  const int row0 = tile * S::BM;
+  run_paged_tile<T, D, PP, PagedSplitRows>(
+      a, qlen * G - row0, row0, [=](const auto& args, PagedSplitRows& P) {
+        paged_rows(args, hk, b, qs, qlen, P);
+        const int chunk = ((P.seq_len + nsplit - 1) / nsplit + 127) / 128 * 128;
+        P.split_lo = split * chunk;
+        P.split_hi = P.split_lo + chunk;
+        const int64_t origin =
+            ((int64_t)split * args.num_heads + (int64_t)hk * (args.num_heads / args.num_kv_heads)) *
+                args.num_tokens + qs;
+        P.po = po + origin * D;
+        P.plse = plse + origin;
+        P.p_head = args.num_tokens;
+        P.D = D;
+      });
 }
 
 // Merges the nsplit partials of each (query head, token): O = sum_s w_s O_s /
@@ -520,9 +591,8 @@ __global__ __launch_bounds__(256) void paged_combine_kernel(fa_paged_args a, int
 // workgroup per 32 query rows of a head.
 template <class T, int D>
 static hipError_t launch_dense_split(const fa_fwd_args& a, int mode, hipStream_t st) {
-  using S = FwdSplitShape<D>;
   const dim3 grid((unsigned)((a.seqlen_q + 31) / 32) * a.num_heads * a.batch),
-      block(64 * S::NW);
+      block(64 * dense_split_waves(D));
   if (mode == kMaskCausal)
     hipLaunchKernelGGL((fwd_split_kernel<T, D, kMaskCausal>), grid, block, 0, st, a);
   else if (mode == kMaskBand)

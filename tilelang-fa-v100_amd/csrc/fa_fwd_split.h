@@ -1,5 +1,7 @@
-// Dense attention forward for problems whose query tiles cannot fill the GPU
-// (gfx950): keys split across the waves of a workgroup.
+// Attention forward of a 32-row query tile with its keys split across the
+// waves of a workgroup (gfx950): dense problems whose query tiles cannot fill
+// the GPU, and paged tiles of at most 32 rows (decoding sequences in a
+// prefill batch).
 //
 // Same mathematics as the other forward cores (the reference's
 // _forward_lse_kernel_func, tilelang_fa_v100/_kernels_forward.py:94-172):
@@ -27,10 +29,10 @@
 
 namespace fa {
 
-template <int D_>
+template <int D_, int NW_>
 struct FwdSplitShape {
   static constexpr int D = D_;
-  static constexpr int NW = D == 64 ? tiles::kFwdSplitWaves64 : tiles::kFwdSplitWaves128;
+  static constexpr int NW = NW_;                 // waves, each with its own keys
   static constexpr int BK = 32;                  // keys per tile
   static constexpr int ROWB = 2 * D;             // bytes per K / V row
   static constexpr int CPR = D / 8;              // 16-byte chunks per row
@@ -46,49 +48,40 @@ struct FwdSplitShape {
   static constexpr int MERGE = NW * 32 * OPS * 4 + 2 * NW * 32 * 4;
   static constexpr int LDS = NW * WAVEB > MERGE ? NW * WAVEB : MERGE;
   static constexpr int SWZ = CPR >= 16 ? 15 : CPR - 1;  // chunk swizzle bits
-  static_assert((D == 64 || D == 128) && BLKS * 1024 == TILEB, "shape");
+  static_assert((D == 64 || D == 128 || D == 256) && BLKS * 1024 == TILEB, "shape");
   static_assert(LDS <= 160 * 1024, "LDS");
   static_assert(32 % NW == 0 && 64 % (32 / NW) == 0 && D % (64 / (32 / NW)) == 0 &&
                     (D / (64 / (32 / NW))) % 2 == 0,
                 "merge split");
 };
 
-template <class T, int D_, int MODE>
-__global__ __launch_bounds__(64 * FwdSplitShape<D_>::NW) void fwd_split_kernel(fa_fwd_args a) {
-  using S = FwdSplitShape<D_>;
+// One 32-row query tile of problem P (rows row0 .. row0 + 31): keys split over
+// the workgroup's NW waves.  Prob as for attn_fwd_tile (fa_fwd_core.h); K / V
+// rows are either row-strided (dense) or in pages of at least 16 keys.
+template <class T, int D_, int NW_, class Prob>
+__device__ __forceinline__ void attn_fwd_split_tile(const Prob& P, int row0, float scale,
+                                                    char* smem) {
+  using S = FwdSplitShape<D_, NW_>;
   constexpr int D = S::D, NW = S::NW, ROWB = S::ROWB;
-  __shared__ __attribute__((aligned(16))) char smem[S::LDS];
   constexpr float kLazy = 8.f;
 
-  const int Sq = a.seqlen_q, Sk = a.seqlen_k, H = a.num_heads;
-  const int nblk = (Sq + 31) / 32;
-  const TileHead th = xcd_tile_order(blockIdx.x, nblk, a.batch * H);
-  const int bh = th.bh, h = bh % H, b = bh / H;
-  const int hk = h / (H / a.num_heads_k);
-  const int row0 = 32 * th.rank;
-  const Band band = mode_band<MODE>(a);
-  auto kv_lo = [&](int r) { return band.wl >= 0 ? min(max(r + band.off - band.wl, 0), Sk) : 0; };
-  auto kv_hi = [&](int r) {
-    return band.wr >= 0 ? min(max(r + band.off + band.wr + 1, 0), Sk) : Sk;
-  };
-
+  const int nrows = P.nrows;
   const int lane = threadIdx.x & 63, wave = wave_id();
   const int lr = lane & 31, lh = lane >> 5;
-  const float scale_log2 = a.softmax_scale * kLog2e;
+  const float scale_log2 = scale * kLog2e;
 
-  const int row_last = min(row0 + 31, Sq - 1);
+  const int row_last = min(row0 + 31, nrows - 1);
   const int row = row0 + lr;
-  const bool row_valid = row < Sq;
-  const int my_lo = row_valid ? kv_lo(row) : 0, my_hi = row_valid ? kv_hi(row) : 0;
+  const bool row_valid = row < nrows;
+  const int my_lo = row_valid ? P.kv_lo(row) : 0, my_hi = row_valid ? P.kv_hi(row) : 0;
   // The keys any row of the block sees, [k_lo, k_hi), in NW ranges of whole
   // 32-key tiles; this wave's tiles are [t0, t1).
-  const int k_lo = kv_lo(row0) / 32 * 32, k_hi = kv_hi(row_last);
+  const int k_lo = __builtin_amdgcn_readfirstlane(P.kv_lo(row0) / 32 * 32);
+  const int k_hi = __builtin_amdgcn_readfirstlane(P.kv_hi(row_last));
+  const int lo_last = P.kv_lo(row_last), hi_first = P.kv_hi(row0);
   const int ntiles = max((k_hi - k_lo + 31) / 32, 0);
   const int per = (ntiles + NW - 1) / NW;
   const int t0 = min(wave * per, ntiles), t1 = min(t0 + per, ntiles);
-
-  const uint16_t* kg = static_cast<const uint16_t*>(a.k) + b * a.k_stride[0] + hk * a.k_stride[2];
-  const uint16_t* vg = static_cast<const uint16_t*>(a.v) + b * a.v_stride[0] + hk * a.v_stride[2];
 
   // ---- wave-private tiles: [buffer][K, V][32 rows][ROWB], chunk c of row r
   // stored at chunk c ^ swz(r).
@@ -96,20 +89,45 @@ __global__ __launch_bounds__(64 * FwdSplitShape<D_>::NW) void fwd_split_kernel(f
   auto kbuf = [&](int bf) { return wbase + bf * 2 * S::TILEB; };  // bf < NBUF
   auto vbuf = [&](int bf) { return wbase + bf * 2 * S::TILEB + S::TILEB; };
   auto swz = [](int r) { return swz_chunk(r) & S::SWZ; };
-  // DMA of tile t (keys k_lo + 32t ..): lane l of block blk holds row
-  // RPB blk + l / CPR, stored chunk l % CPR; rows past the last key repeat it
-  // (their scores are masked).
-  auto issue = [&](int t, int bf) {
+  // DMA of the K or V rows of tile t (keys k_lo + 32t ..): lane l of block blk
+  // holds row RPB blk + l / CPR, stored chunk l % CPR; rows past the last key
+  // any row sees repeat it (their scores are masked).
+  constexpr int HB = S::BLKS / 2;  // blocks per 16 rows
+  uint32_t k_loff[HB], v_loff[HB];  // paged: element offsets within 16 rows of a page
+  if constexpr (!Prob::kRowStrided) {
+#pragma unroll
+    for (int i = 0; i < HB; ++i) {
+      const uint32_t r = S::RPB * i + lane / S::CPR;
+      const uint32_t c = 8 * ((lane % S::CPR) ^ swz(r));
+      k_loff[i] = r * (uint32_t)P.k_row_stride() + c;
+      v_loff[i] = r * (uint32_t)P.v_row_stride() + c;
+    }
+  }
+  auto issue_rows = [&](int t, char* dst, auto is_v) {
+    constexpr bool kV = decltype(is_v)::value;
     const int n0 = k_lo + 32 * t;
+    if (!Prob::kRowStrided && n0 + 32 <= k_hi) {
+      // Whole tile of a paged problem: 16 rows from one page, whose base is
+      // wave-uniform (scalar block-table loads).
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf) {
+        const uint16_t* base = kV ? P.v_ptr(n0 + 16 * hf) : P.k_ptr(n0 + 16 * hf);
+#pragma unroll
+        for (int i = 0; i < HB; ++i)
+          global_lds16_opaque(base + (kV ? v_loff[i] : k_loff[i]), dst + (HB * hf + i) * 1024);
+      }
+      return;
+    }
 #pragma unroll
     for (int blk = 0; blk < S::BLKS; ++blk) {
       const int r = S::RPB * blk + lane / S::CPR;
       const int c = (lane % S::CPR) ^ swz(r);
-      const int64_t n = min(n0 + r, Sk - 1);
-      global_lds16_opaque(kg + n * a.k_stride[1] + 8 * c, kbuf(bf) + blk * 1024);
-      global_lds16_opaque(vg + n * a.v_stride[1] + 8 * c, vbuf(bf) + blk * 1024);
+      const int n = min(n0 + r, k_hi - 1);
+      global_lds16_opaque((kV ? P.v_ptr(n) : P.k_ptr(n)) + 8 * c, dst + blk * 1024);
     }
   };
+  auto issue_k = [&](int t, int bf) { issue_rows(t, kbuf(bf), BoolC<false>{}); };
+  auto issue_v = [&](int t, int bf) { issue_rows(t, vbuf(bf), BoolC<true>{}); };
   // K operand of Sᵀ = K Qᵀ, chunk c: row lr, logical chunk 2c + lh.
   int koff[D / 16];
 #pragma unroll
@@ -136,18 +154,20 @@ __global__ __launch_bounds__(64 * FwdSplitShape<D_>::NW) void fwd_split_kernel(f
   float ms_run = neg_inf(), l_run = 0.f;
   u32x4 qf[D / 16];  // the lane's query row (B operand chunks), loaded below
 
-  auto compute = [&](int t, int bf) {
-    const int n0 = k_lo + 32 * t;
+  f32x16 s;
+  auto scores = [&](int bf) {
     const char* kb = kbuf(bf);
-    const char* vb = vbuf(bf);
-    f32x16 s;
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = 0.f;
 #pragma unroll
     for (int c = 0; c < D / 16; ++c) s = T::mma32(ld16(kb + koff[c]), qf[c], s);
+  };
+  u32x4 pb[2];
+  auto softmax = [&](int t) {
+    const int n0 = k_lo + 32 * t;
     // Element i is key n0 + 8(i/4) + 4lh + i%4 of the lane's row (rows past
-    // Sq compute garbage that the merge never stores).
-    if (n0 < kv_lo(row_last) || n0 + 32 > kv_hi(row0)) {
+    // the last compute garbage that the merge never stores).
+    if (n0 < lo_last || n0 + 32 > hi_first) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const int kv = n0 + 8 * (i >> 2) + 4 * lh + (i & 3);
@@ -172,7 +192,6 @@ __global__ __launch_bounds__(64 * FwdSplitShape<D_>::NW) void fwd_split_kernel(f
         for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
     }
     const float mb = ms_run == neg_inf() ? 0.f : ms_run;
-    u32x4 pb[2];
 #pragma unroll
     for (int kc = 0; kc < 2; ++kc)
 #pragma unroll
@@ -181,8 +200,16 @@ __global__ __launch_bounds__(64 * FwdSplitShape<D_>::NW) void fwd_split_kernel(f
         const float p0 = fast_exp2(fmaf(s[e], scale_log2, -mb));
         const float p1 = fast_exp2(fmaf(s[e + 1], scale_log2, -mb));
         pb[kc][w] = T::pack(p0, p1);
-        l_run = T::sum2(p0, p1, pb[kc][w], l_run);
+        // Paged tiles sum the fp32 values, as the row-tile core they stand in
+        // for does; the dense kernel the rounded ones (fp16: one v_dot2).
+        if constexpr (Prob::kRowStrided)
+          l_run = T::sum2(p0, p1, pb[kc][w], l_run);
+        else
+          l_run = l_run + (p0 + p1);
       }
+  };
+  auto accumulate = [&](int bf) {
+    const char* vb = vbuf(bf);
 #pragma unroll
     for (int kc = 0; kc < 2; ++kc)
 #pragma unroll
@@ -192,38 +219,64 @@ __global__ __launch_bounds__(64 * FwdSplitShape<D_>::NW) void fwd_split_kernel(f
         o[dt] = T::mma32(u32x4{lo[0], lo[1], hi[0], hi[1]}, pb[kc], o[dt]);
       }
   };
+  // Waits for all but the n newest DMAs, and for the operand reads issued so
+  // far before their buffer is overwritten.
+  auto wait_but = [](auto n) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(n)::value) : "memory");
+  };
+  auto wait_reads = []() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
 
-  // ---- the wave's key loop: tile t in buffer (t - t0) % 2; the DMA of tile
-  // t + 1 is in flight while tile t is computed (2 BLKS DMAs per tile).
-  if (t0 < t1) issue(t0, 0);
-  // The lane's query row as B operand chunks (zero for rows past Sq), loaded
-  // while the first tile is in flight; one wait covers both, so the
+  if (t0 < t1) {
+    issue_k(t0, 0);
+    issue_v(t0, 0);
+  }
+  // The lane's query row as B operand chunks (zero for rows past the last),
+  // loaded while the first tile is in flight; one wait covers both, so the
   // compiler's own wait before the first product (it does not see the DMA)
   // cannot also wait for the next tile's.
   {
-    const uint16_t* qp = static_cast<const uint16_t*>(a.q) + b * a.q_stride[0] +
-                         h * a.q_stride[2] + (int64_t)min(row, Sq - 1) * a.q_stride[1];
+    const uint16_t* qp = row_valid ? P.q_ptr(row) : nullptr;
 #pragma unroll
     for (int c = 0; c < D / 16; ++c)
       qf[c] = row_valid ? ld16(qp + 16 * c + 8 * lh) : u32x4{0, 0, 0, 0};
   }
-  wait_vmem();
-  for (int t = t0; t < t1; ++t) {
-    const int bf = S::NBUF == 2 ? (t - t0) & 1 : 0;
-    if (S::NBUF == 2 && t + 1 < t1) {
-      issue(t + 1, bf ^ 1);
-      if constexpr (2 * S::BLKS == 8)
-        __builtin_amdgcn_s_waitcnt(0x0F78);  // vmcnt(8): tile t landed
-      else
-        __builtin_amdgcn_s_waitcnt(0x4F70);  // vmcnt(16)
-    } else {
-      wait_vmem();
+  wait_but(IntC<0>{});
+  if constexpr (S::NBUF == 2) {
+    // Tile t in buffer (t - t0) % 2; the DMA of tile t + 1 is in flight while
+    // tile t is computed (2 BLKS DMAs per tile).
+    for (int t = t0; t < t1; ++t) {
+      const int bf = (t - t0) & 1;
+      if (t + 1 < t1) {
+        issue_k(t + 1, bf ^ 1);
+        issue_v(t + 1, bf ^ 1);
+        wait_but(IntC<2 * S::BLKS>{});
+      } else {
+        wait_but(IntC<0>{});
+      }
+      scores(bf);
+      softmax(t);
+      accumulate(bf);
+      wait_reads();
     }
-    compute(t, bf);
-    // The next DMA into this buffer is issued after the operand reads of
-    // this tile have returned.
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-    if (S::NBUF == 1 && t + 1 < t1) issue(t + 1, 0);
+  } else {
+    // One buffer: K(t + 1) is requested once the scores of tile t have read
+    // K(t), V(t + 1) once its products have read V(t), so each is in flight
+    // for the other half of the tile's work.
+    for (int t = t0; t < t1; ++t) {
+      const bool more = t + 1 < t1;
+      if (t > t0) wait_but(IntC<S::BLKS>{});  // K(t) landed, V(t) may be in flight
+      scores(0);
+      wait_reads();
+      if (more) issue_k(t + 1, 0);
+      softmax(t);
+      if (more)
+        wait_but(IntC<S::BLKS>{});  // V(t) landed, K(t + 1) may be in flight
+      else
+        wait_but(IntC<0>{});
+      accumulate(0);
+      wait_reads();
+      if (more) issue_v(t + 1, 0);
+    }
   }
 
   // ---- merge.  Each wave's partial for its 32 rows: O (fp32, unnormalised
@@ -272,15 +325,19 @@ __global__ __launch_bounds__(64 * FwdSplitShape<D_>::NW) void fwd_split_kernel(f
       }
     }
   }
-  if (orow_g >= Sq) return;
+  if (orow_g >= nrows) return;
   const float inv = L > 0.f ? 1.f / L : 0.f;
-  uint16_t* dst = static_cast<uint16_t*>(a.out) + b * a.o_stride[0] + h * a.o_stride[2] +
-                  (int64_t)orow_g * a.o_stride[1] + d0;
+  auto* dst = fwd_out_ptr(P, orow_g, d0);
 #pragma unroll
-  for (int j = 0; j < DPL; j += 2)
-    *reinterpret_cast<uint32_t*>(dst + j) = T::pack(acc[j] * inv, acc[j + 1] * inv);
-  if (a.lse && lane % LPR == 0)
-    a.lse[(int64_t)bh * Sq + orow_g] = L > 0.f ? (M + log2f(L)) * kLn2 : neg_inf();
+  for (int j = 0; j < DPL; j += 2) {
+    if constexpr (Prob::kF32Out)
+      *reinterpret_cast<float2*>(dst + j) = float2{acc[j] * inv, acc[j + 1] * inv};
+    else
+      *reinterpret_cast<uint32_t*>(dst + j) = T::pack(acc[j] * inv, acc[j + 1] * inv);
+  }
+  float* lp = fwd_lse_ptr(P, orow_g);
+  if (lp != nullptr && lane % LPR == 0)
+    *lp = L > 0.f ? (M + log2f(L)) * (Prob::kF32Out ? 1.f : kLn2) : neg_inf();
 }
 
 }  // namespace fa
