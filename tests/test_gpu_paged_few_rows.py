@@ -39,3 +39,25 @@ def test_few_row_tiles_match_oracle(case):
     c = make_case(29, ql, sl, [s - q for q, s in zip(ql, sl)], Hq, Hkv, D, page=page, dtype=dt)
     print(f"case {case}", flush=True)
     run_split(c, ns, causal=causal, wq=wq, wk=wk)
+
+
+@pytest.mark.parametrize("Hkv,splits", [(1, 1), (2, 1), (2, 3), (3, 1), (4, 2), (5, 1), (8, 2),
+                                        (12, 1), (16, 1)])
+def test_workgroup_order_covers_every_tile(Hkv, splits):
+    """Every (KV head, key range) count of the workgroup order: more than,
+    fewer than and no divisor of the 8 XCDs."""
+    c = make_case(31, [300, 1, 0, 40, 257], [300, 77, 9, 640, 300], [0, 76, 9, 600, 43],
+                  Hkv, Hkv, 128, page=16)
+    run_split(c, splits)
+
+
+@pytest.mark.parametrize("q_lens,heads", [
+    ([1] * 20 + [600] * 9, 32),           # 65 tiles x 32 heads: sequences by history
+    ([1, 2, 129, 64, 0, 300] * 10, 4),    # 60 sequences, tiles by reach, many ties
+    ([3, 1, 130, 0, 1] * 14, 4),          # 70 sequences: scanned in their own order
+], ids=["by-history", "by-reach", "over-64"])
+def test_tile_orders_cover_every_tile(q_lens, heads):
+    g = torch.Generator().manual_seed(37)
+    pf = torch.randint(0, 5, (len(q_lens),), generator=g).mul(50).tolist()
+    c = make_case(33, q_lens, [p + q for p, q in zip(pf, q_lens)], pf, heads, heads, 64, page=16)
+    run_split(c, 1)

@@ -578,14 +578,4 @@ __device__ __forceinline__ const __attribute__((address_space(4))) Args* kernel_
   return p;
 }
 
-// XCD-aware workgroup order.  The hardware hands consecutive workgroup ids to
-// the 8 XCDs round-robin; remapping makes each XCD receive a contiguous range
-// of logical tiles, so tiles that share K/V rows share one L2.
-__device__ __forceinline__ int xcd_remap(int linear, int total) {
-  constexpr int kXcds = 8;
-  if (total % kXcds != 0) return linear;
-  const int per = total / kXcds;
-  return (linear % kXcds) * per + linear / kXcds;
-}
-
 }  // namespace fa

@@ -291,66 +291,108 @@ struct PagedSplitRows : PagedRows {
   }
 };
 
-// Finds the sequence owning `tile` in the varlen tile space where sequence b
-// has ceil(qlen_b * G / BM) tiles.  Returns b (or -1) and the tile index
-// within the sequence.  Wave 0 scans the sequences 64 at a time with a
-// shuffle prefix sum and finds the owner with a ballot; one barrier hands
-// the result to the other waves (a block-wide scan in LDS took 16
-// barriers).  Up to 64 sequences are taken in order of decreasing history
-// (prefix_kv_lens; equal histories keep their order): a sequence's tiles all
-// see about its history plus its own length in keys, so with the
-// heaviest-first order inside each sequence the tiles go out roughly
-// longest first, and the last workgroups on each CU are short (C5, chunked
-// prefill with histories of 0-8k keys: 2% faster; 5% less idle time in a
-// dispatch simulation, part of it spent on the sort).  When all histories
-// are equal the order is the sequences' own.
+// Workgroup order of the paged kernels: `combos` (KV head, key range) pairs x
+// row-tile slots, slot 0 the tile with the most keys (find_sequence).  The
+// hardware deals workgroup ids to the 8 XCDs in turn and starts each XCD's in
+// order, so every XCD gets whole combos where they divide evenly (its tiles
+// share K / V in its L2), or shares a combo's slots with others in turn where
+// there are fewer, and always walks the slots from the first: long tiles start
+// first on every XCD and in every combo.  Ranges of ids that were contiguous
+// per XCD (combo-major) started each combo's long tiles when the one before
+// it ended, and with 1, 2 or 4 KV heads gave some XCDs only the long tiles and
+// others the short ones (figures at tiles::kPagedTileOrderMax).
+struct SlotCombo {
+  int slot, combo, combo_count;
+};
+constexpr int kOrderXcds = 8;
+__device__ __forceinline__ SlotCombo paged_order(int wg, int combos) {
+  const int x = wg % kOrderXcds, l = wg / kOrderXcds;
+  if (combos % kOrderXcds == 0) {
+    const int per = combos / kOrderXcds;
+    return {l / per, x * per + l % per, combos};
+  }
+  if (kOrderXcds % combos == 0) {
+    return {l * (kOrderXcds / combos) + x / combos, x % combos, combos};
+  }
+  return {wg / combos, wg % combos, combos};
+}
+// Workgroups that cover `slots` slots of `combos` combos (slots past the last
+// tile find no sequence).
+static int64_t paged_order_grid(int64_t slots, int64_t combos) {
+  const int64_t f = kOrderXcds % combos == 0 ? kOrderXcds / combos : 1;
+  return (slots + f - 1) / f * f * combos;
+}
+
+// Inclusive prefix sum over the 64 lanes: DPP adds within rows of 16, then
+// row broadcasts (a shuffle goes through LDS, ~10 times the latency).
+__device__ __forceinline__ int wave_scan(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);  // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);  // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);  // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);  // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, true);  // row_bcast:15
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, true);  // row_bcast:31
+  return x;
+}
+__device__ __forceinline__ int wave_total(int x) {
+  return __builtin_amdgcn_readlane(wave_scan(x), 63);
+}
+
+// Finds the sequence owning slot `tile` in the varlen tile space where
+// sequence b has ceil(qlen_b * G / BM) tiles.  Returns b (or -1) and the
+// tile's index from the sequence's last (the one that sees most keys).
+// Up to 64 sequences, one per lane of wave 0, in one of two orders; u_b is the
+// history in units of a tile's rows, u_b + i + 1 the reach of tile i:
+//  * grids of few rounds (tiles x combos up to kPagedTileOrderMax): all tiles by
+//    decreasing reach, ties by sequence.  Sequence b has n_b(K) = clamp(u_b +
+//    ntiles_b - K, 0, ntiles_b) tiles of reach above K;
+//  * larger grids: sequences by decreasing history (the tiles of one share its
+//    K / V in the L2, and the tail is a small part), n_b(K) = all or none.
+// Either way a binary search for the smallest K with at most `tile` tiles above
+// it, and the slot's rank among those at K, name the tile.  More sequences are
+// scanned in their own order, 64 at a time.
 __device__ int find_sequence(const int32_t* qsl, const int32_t* prefix, int batch, int G,
-                             int BM, int tile, int* local) {
+                             int BM, int combos, int tile, int* local) {
   __shared__ int found_b, found_local;
   if (wave_id() == 0) {
     const int lane = threadIdx.x & 63;
-    int base = 0, fb = -1, fl = 0;
-    // The sort costs wave 0 about a microsecond of dependent shuffles; it is
-    // skipped when the histories are all equal (the order would not change).
-    const bool sort = batch <= 64 &&
-                      __ballot(lane < batch && prefix[lane] != prefix[0]) != 0;
-    if (sort) {
-      // Bitonic sort of (history descending, index ascending) across lanes;
-      // lanes past the batch sort last.
-      const uint32_t hist = lane < batch ? (uint32_t)max(prefix[lane], 0) : 0u;
-      uint64_t key = lane < batch ? ((uint64_t)(0x7fffffffu - hist) << 32) | (uint32_t)lane
-                                  : ~0ull;
-#pragma unroll
-      for (int k = 2; k <= 64; k <<= 1)
-#pragma unroll
-        for (int j = k >> 1; j > 0; j >>= 1) {
-          const uint64_t other = ((uint64_t)(uint32_t)__shfl_xor((int)(key >> 32), j) << 32) |
-                                 (uint32_t)__shfl_xor((int)(uint32_t)key, j);
-          const bool up = (lane & k) == 0, lower = (lane & j) == 0;
-          const uint64_t lo = key < other ? key : other, hi = key < other ? other : key;
-          key = (up == lower) ? lo : hi;
-        }
-      const int sb = key == ~0ull ? batch : (int)(uint32_t)key;  // sequence at this lane
-      int n = 0;
-      if (sb < batch) {
-        const int ql = qsl[sb + 1] - qsl[sb];
+    int fb = -1, fl = 0;
+    if (batch <= 64) {
+      int n = 0, u = 0;
+      if (lane < batch) {
+        const int ql = qsl[lane + 1] - qsl[lane];
         n = ql > 0 ? (int)(((int64_t)ql * G + BM - 1) / BM) : 0;
+        u = (int)min((int64_t)max(prefix[lane], 0) * G / BM, (int64_t)1 << 29);
       }
-      int incl = n;
-#pragma unroll
-      for (int off = 1; off < 64; off <<= 1) {
-        const int v = __shfl_up(incl, off);
-        if (lane >= off) incl += v;
+      const bool by_tile =
+          (int64_t)wave_total(n) * combos <= (int64_t)tiles::kPagedTileOrderMax;
+      auto above = [&](int K) {
+        return by_tile ? min(max(u + n - K, 0), n) : (u > K ? n : 0);
+      };
+      // lo: more than `tile` tiles above it (or -1); hi: at most `tile`.
+      int lo = -1, hi = 1;
+      while (wave_total(above(hi)) > tile) {
+        lo = hi;
+        hi *= 2;
       }
-      const int excl = incl - n;
-      const bool hit = sb < batch && n > 0 && tile >= excl && tile < incl;
-      const uint64_t m = __ballot(hit);
-      if (m) {
-        const int src = __ffsll((unsigned long long)m) - 1;
-        fb = __shfl(sb, src);
-        fl = tile - __shfl(excl, src);
+      while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (wave_total(above(mid)) > tile)
+          lo = mid;
+        else
+          hi = mid;
+      }
+      const int before = above(hi);
+      const int rank = tile - wave_total(before);  // among the tiles at K = hi
+      const int here = above(hi - 1) - before;
+      const int last = wave_scan(here);
+      const uint64_t hit = __ballot(here > 0 && rank >= last - here && rank < last);
+      if (hit) {
+        fb = __ffsll((unsigned long long)hit) - 1;
+        fl = __builtin_amdgcn_readlane(before + rank - (last - here), fb);
       }
     } else {
+      int base = 0;
       for (int c0 = 0; c0 < batch; c0 += 64) {
         const int b = c0 + lane;
         int n = 0;
@@ -472,13 +514,12 @@ __global__ __launch_bounds__((FwdKernelCfg<D, PP>::THREADS), (FwdKernelCfg<D, PP
 void fwd_paged_kernel(fa_paged_args a) {
   using S = FwdKernelCfg<D, PP>;
   const int G = a.num_heads / a.num_kv_heads;
-  const int slots = gridDim.x / a.num_kv_heads;
-  const int id = xcd_remap(blockIdx.x, gridDim.x);
-  const int hk = id / slots;
-  const int slot = id % slots;
+  const SlotCombo sc = paged_order(blockIdx.x, a.num_kv_heads);
+  const int hk = sc.combo, slot = sc.slot;
 
   int local = 0;
-  const int b = find_sequence(a.query_start_loc, a.prefix_kv_lens, a.batch, G, S::BM, slot, &local);
+  const int b = find_sequence(a.query_start_loc, a.prefix_kv_lens, a.batch, G, S::BM,
+                              sc.combo_count, slot, &local);
   if (b < 0) return;
   const int qs = a.query_start_loc[b];
   const int qlen = a.query_start_loc[b + 1] - qs;
@@ -491,24 +532,21 @@ void fwd_paged_kernel(fa_paged_args a) {
       [=](const auto& args, PagedRows& P) { paged_rows(args, hk, b, qs, qlen, P); });
 }
 
-// Split-KV variant: workgroup (split, KV head, tile slot); the splits of a
+// Split-KV variant: workgroup (KV head, split, tile slot); the splits of a
 // sequence cover its keys in ranges of ceil(seq_len / nsplit) rounded up to
-// 128.  Consecutive workgroup ids share the split and KV head (the same
-// K / V pages).
+// 128.
 template <class T, int D, bool PP>
 __global__ __launch_bounds__((FwdKernelCfg<D, PP>::THREADS), (FwdKernelCfg<D, PP>::WAVES_PER_EU))
 void fwd_paged_split_kernel(fa_paged_args a, int nsplit, float* po, float* plse) {
   using S = FwdKernelCfg<D, PP>;
   const int G = a.num_heads / a.num_kv_heads;
-  const int per_split = gridDim.x / nsplit;
-  const int slots = per_split / a.num_kv_heads;
-  const int id = xcd_remap(blockIdx.x, gridDim.x);
-  const int split = id / per_split;
-  const int hk = (id % per_split) / slots;
-  const int slot = id % slots;
+  const SlotCombo sc = paged_order(blockIdx.x, a.num_kv_heads * nsplit);
+  const int hk = sc.combo / nsplit, split = sc.combo % nsplit;
+  const int slot = sc.slot;
 
   int local = 0;
-  const int b = find_sequence(a.query_start_loc, a.prefix_kv_lens, a.batch, G, S::BM, slot, &local);
+  const int b = find_sequence(a.query_start_loc, a.prefix_kv_lens, a.batch, G, S::BM,
+                              sc.combo_count, slot, &local);
   if (b < 0) return;
   const int qs = a.query_start_loc[b];
   const int qlen = a.query_start_loc[b + 1] - qs;
@@ -672,16 +710,17 @@ int paged_grid_slots(const fa_paged_args& a) {
 template <class T, int D, bool PP>
 static hipError_t launch_paged_pp(const fa_paged_args& a, int nsplit, void* ws,
                                   hipStream_t st) {
-  const unsigned slots = (unsigned)paged_grid_slots(a) * a.num_kv_heads;
+  const unsigned grid = (unsigned)paged_order_grid(
+      paged_grid_slots(a), (int64_t)a.num_kv_heads * std::max(nsplit, 1));
   if (nsplit <= 1) {
-    hipLaunchKernelGGL((fwd_paged_kernel<T, D, PP>), dim3(slots),
+    hipLaunchKernelGGL((fwd_paged_kernel<T, D, PP>), dim3(grid),
                        dim3(FwdKernelCfg<D, PP>::THREADS), 0, st, a);
     return hipGetLastError();
   }
   const size_t rows = (size_t)nsplit * a.num_heads * a.num_tokens;
   float* po = static_cast<float*>(ws);
   float* plse = po + rows * D;
-  hipLaunchKernelGGL((fwd_paged_split_kernel<T, D, PP>), dim3(slots * (unsigned)nsplit),
+  hipLaunchKernelGGL((fwd_paged_split_kernel<T, D, PP>), dim3(grid),
                      dim3(FwdKernelCfg<D, PP>::THREADS), 0, st, a, nsplit, po, plse);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
@@ -727,22 +766,28 @@ size_t paged_split_workspace_bytes(const fa_paged_args& a, int nsplit) {
   return rows * a.head_dim * sizeof(float) + rows * sizeof(float) + 256;
 }
 
-// Split count from sizes alone (no device data): split only when the query
-// tiles cannot occupy the GPU (fewer workgroups than CUs) and the block
-// table can hold long sequences; each split covers at least 2048 keys.
+// Split count from sizes alone (no device data).  Workgroups unsplit: the row
+// tiles of all tokens together, but at least one per sequence (every sequence
+// with tokens has a tile of its own), times the KV heads.
 int paged_num_splits(const fa_paged_args& a) {
   const int G = a.num_heads / a.num_kv_heads;
-  const int64_t tiles =
-      ((int64_t)a.num_tokens * G + paged_block_rows(a) - 1) / paged_block_rows(a);
-  const int64_t wgs = std::max<int64_t>(1, tiles * a.num_kv_heads);
+  const int64_t rows = (int64_t)a.num_tokens * G;
+  const int64_t seqs = std::max(1, std::min(a.batch, a.num_tokens));
+  const int64_t tiles = std::max<int64_t>(
+      seqs, (rows + paged_block_rows(a) - 1) / paged_block_rows(a));
+  const int64_t wgs = tiles * a.num_kv_heads;
   const int64_t kv_cap = (int64_t)a.max_blocks * a.page_size;
   const int cus = device_cu_count();
-  if (wgs >= cus || kv_cap < tiles::kSplitMinKeys) return 1;
-  // About one workgroup per CU, and no range longer than kSplitMaxRangeKeys
-  // (a workgroup's serial length), but none shorter than kSplitMinRangeKeys
-  // (each split adds a partial O per row to write and merge).
-  int64_t ns = std::max<int64_t>((cus + wgs - 1) / wgs,
-                                 (kv_cap + tiles::kSplitMaxRangeKeys - 1) / tiles::kSplitMaxRangeKeys);
+  if (kv_cap < tiles::kSplitMinKeys || 2 * wgs >= 3 * cus) return 1;
+  // Below 1.5 workgroups per CU no range is longer than kSplitMaxRangeKeys (a
+  // workgroup's serial length); below one, about one workgroup per CU, or two
+  // where the tiles hold few rows (tiles bound by latency, whose partials are
+  // small); never shorter than kSplitMinRangeKeys (each split adds a partial O
+  // per row to write and merge).
+  int64_t ns = (kv_cap + tiles::kSplitMaxRangeKeys - 1) / tiles::kSplitMaxRangeKeys;
+  const bool few = rows <= 32 * seqs;
+  const int64_t want = few ? 2 * cus : cus;
+  if (wgs < cus) ns = std::max<int64_t>(ns, (want + wgs - 1) / wgs);
   ns = std::min<int64_t>(ns, kv_cap / tiles::kSplitMinRangeKeys);
   return (int)std::max<int64_t>(1, std::min<int64_t>(ns, kMaxPagedSplits));
 }

@@ -165,20 +165,39 @@ constexpr int kDecTilesInFlight = 2;
 constexpr int kDecChunkElems = 32768;
 
 // ---- split-KV paged prefill (fa_fwd.hip paged_num_splits): no split when
-// the query tiles alone give >= CU-count workgroups or the block table holds
-// fewer than kSplitMinKeys keys; otherwise max(ceil(CUs / workgroups),
-// ceil(keys / kSplitMaxRangeKeys)) ranges, but none shorter than
-// kSplitMinRangeKeys and at most kMaxSplits.
+// the tiles (at least one per sequence) give 1.5 workgroups per CU or the
+// block table holds fewer than kSplitMinKeys keys; otherwise
+// ceil(keys / kSplitMaxRangeKeys) ranges, and below one workgroup per CU at
+// least ceil(CUs / workgroups) (twice that for tiles of few rows), but none
+// shorter than kSplitMinRangeKeys and at most kMaxSplits.
 // Evidence (2 sequences, 32 / 8 heads, D = 128, time per call in ms for
 // 1 / 4 / 8 / 16 splits): 32k-key prefix + 128 tokens 0.955 / 0.277 / 0.171 /
 // 0.192 (this rule: 8); 16k + 128: 0.487 / 0.153 / 0.104 / 0.128 (8);
 // 32k + 512: 0.994 / 0.593 / 0.634 / 0.729 (5); 8k + 64: 0.252 / 0.087 /
 // 0.062 / 0.080 (8).  The former rule (2 x CUs / workgroups ranges of at
 // least 2048 keys) chose 16, 8, 4 and 4.
+// Batches of one-token sequences, 1-8k keys (us for 1 / 2 / 4 / 8): 64 of them
+// 224 / 235 / 248 / 295 (this rule 1; counting only the token rows' tiles it
+// was 8), 16 of them 110 / 75 / 70 / 81 (4; was 8), 16 of four tokens after
+// 2-16k keys 198 / 144 / 120 / 134 (4; was 16); 47 of them with a 512-token
+// chunk, 64 heads 167 / 198 / 229 / 302 (1; was 2); 30 with two chunks, table
+// of 16k keys 162 / 150 / 187 / 243 (2; was 3).
 constexpr int kSplitMinKeys = 4096;
 constexpr int kSplitMinRangeKeys = 1024;
 constexpr int kSplitMaxRangeKeys = 8192;
 constexpr int kMaxSplits = 64;
+
+// ---- workgroup order of the paged kernels (fa_fwd.hip paged_order,
+// find_sequence): up to this many (tile, KV head, key range) workgroups, about
+// 8 rounds of the chip, every tile by its own reach; above it, whole sequences
+// by their history.  Evidence (us, same box, D = 128 unless noted, against
+// combo-major ranges of ids with sequences by history): 8 prompts of 512-4096
+// tokens, 16 / 2 heads 281 -> 255; 8 of 300-2048, 16 / 16 heads 110 -> 96; 8 of
+// 512-2048, 28 / 4 heads, D = 64 149 -> 129; the same after up to 4k keys, 16 / 2
+// heads, D = 256 988 -> 660; 2 chunks + 30 one-token sequences, 2 ranges 158 ->
+// 150.  Above the limit the tile order lost the K / V reuse in the L2: 8 prompts of
+// 512-4096 tokens, 32 / 8 heads (2400 workgroups) 467 -> 474, by history 460.
+constexpr int kPagedTileOrderMax = 2048;
 
 }  // namespace tiles
 }  // namespace fa
