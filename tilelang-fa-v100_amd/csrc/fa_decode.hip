@@ -206,17 +206,23 @@ __global__ __launch_bounds__(256, 2) void decode_split_kernel(fa_decode_args a,
   }
 }
 
-// One wave per (sequence, query head): merge the chunk partials with weights
-// exp2(lse_c - max), computed lane-parallel, then an unrolled weighted sum.
+// One workgroup of kCombineWaves waves per (sequence, query head): merge the
+// chunk partials with weights exp2(lse_c - max), computed lane-parallel, then
+// an unrolled weighted sum.  Bound by the latency of a wave's chain of partial
+// loads (a long sequence has up to 128 of them), so the waves take the
+// partials in turn and their sums meet in LDS.
+constexpr int kCombineWaves = 4;
 template <class T, int D>
-__global__ __launch_bounds__(64) void decode_combine_kernel(fa_decode_args a,
-                                                            DecodeWs ws) {
+__global__ __launch_bounds__(64 * kCombineWaves) void decode_combine_kernel(fa_decode_args a,
+                                                                          DecodeWs ws) {
   const int CH = ws.split_dev ? *ws.split_dev : ws.split;
   constexpr int NP = (D + 127) / 128;  // d pairs per lane: 2*lane + 128*k
-  __shared__ float wts[64];
+  constexpr int NW = kCombineWaves;
+  __shared__ float wts[NW][64];
+  __shared__ __attribute__((aligned(8))) float part[NW][D];
   const int hq = blockIdx.x % a.num_heads;
   const int b = blockIdx.x / a.num_heads;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63, wave = wave_id();
   const int seq_len = max(0, min(a.seq_lens[b], a.max_blocks * a.page_size));
   const int ns = (seq_len + CH - 1) / CH;
   const int64_t row0 = ((int64_t)b * a.num_heads + hq) * ws.nsplit;
@@ -227,17 +233,16 @@ __global__ __launch_bounds__(64) void decode_combine_kernel(fa_decode_args a,
   float acc[NP][2];
 #pragma unroll
   for (int k = 0; k < NP; ++k) acc[k][0] = acc[k][1] = 0.f;
-  float wsum = 0.f;
+  float wsum = 0.f;  // the same in every wave
   for (int c0 = 0; c0 < ns; c0 += 64) {
     const int cn = min(64, ns - c0);
     const float w = lane < cn ? fast_exp2(ws.plse[row0 + c0 + lane] - m_use) : 0.f;
     wsum += wave_sum(w);
-    wts[lane] = w;
-    __syncthreads();
+    wts[wave][lane] = w;  // each wave its own copy: read back by the same wave only
     const float* base = ws.po + (row0 + c0) * D;
 #pragma unroll 8
-    for (int c = 0; c < cn; ++c) {
-      const float wc = wts[c];
+    for (int c = wave; c < cn; c += NW) {
+      const float wc = wts[wave][c];
 #pragma unroll
       for (int k = 0; k < NP; ++k) {
         const int d = 2 * lane + 128 * k;
@@ -248,18 +253,27 @@ __global__ __launch_bounds__(64) void decode_combine_kernel(fa_decode_args a,
         }
       }
     }
-    __syncthreads();
   }
-  const float inv = wsum > 0.f ? 1.f / wsum : 0.f;
-  uint16_t* op = static_cast<uint16_t*>(a.out) + (int64_t)b * a.o_stride[0] +
-                 (int64_t)hq * a.o_stride[1];
 #pragma unroll
   for (int k = 0; k < NP; ++k) {
     const int d = 2 * lane + 128 * k;
-    if (d < D)
-      *reinterpret_cast<uint32_t*>(op + d) = T::pack(acc[k][0] * inv, acc[k][1] * inv);
+    if (d < D) *reinterpret_cast<float2*>(&part[wave][d]) = float2{acc[k][0], acc[k][1]};
   }
-  if (a.lse && lane == 0)
+  __syncthreads();
+  const float inv = wsum > 0.f ? 1.f / wsum : 0.f;
+  uint16_t* op = static_cast<uint16_t*>(a.out) + (int64_t)b * a.o_stride[0] +
+                 (int64_t)hq * a.o_stride[1];
+  for (int d = 2 * (int)threadIdx.x; d < D; d += 128 * NW) {
+    float2 sum = {0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float2 x = *reinterpret_cast<const float2*>(&part[w][d]);
+      sum.x += x.x;
+      sum.y += x.y;
+    }
+    *reinterpret_cast<uint32_t*>(op + d) = T::pack(sum.x * inv, sum.y * inv);
+  }
+  if (a.lse && threadIdx.x == 0)
     a.lse[(int64_t)b * a.num_heads + hq] =
         wsum > 0.f ? (m_use + log2f(wsum)) * kLn2 : neg_inf();
 }
@@ -298,19 +312,20 @@ static int stream_waves_per_cu(int D) {
   return DecStream<128>::kWavesPerCU;
 }
 
-// Keys per split.  The streaming kernel takes the largest of kSplitMax,
-// kSplitMax / 2, .. kSplitMin whose item count (estimated from max_seq_len)
-// gives every resident wave at least kDecItemsPerWave items.
+// Keys per split.  The streaming kernel takes the largest of kDecSplitKeysMax,
+// half of it, .. kDecSplitKeysMid whose item count (estimated from max_seq_len)
+// gives every resident wave at least kDecItemsPerWave items; where that one
+// gives fewer than one item per two waves, it is halved further, down to
+// kDecSplitKeysMin.
 static int decode_split_size(const fa_decode_args& a) {
   if (!use_stream(a)) return dec_chunk(a.head_dim);
   const int G = a.num_heads / a.num_kv_heads;
   const int64_t heads = (int64_t)a.num_kv_heads * (G / decode_group_size(a));
   const int64_t waves = (int64_t)device_cu_count() * stream_waves_per_cu(a.head_dim);
   int s = tiles::kDecSplitKeysMax;
-  for (; s > tiles::kDecSplitKeysMin; s /= 2) {
-    const int64_t items = (int64_t)a.batch * ((a.max_seq_len + s - 1) / s) * heads;
-    if (items >= tiles::kDecItemsPerWave * waves) break;
-  }
+  auto items = [&](int n) { return (int64_t)a.batch * ((a.max_seq_len + n - 1) / n) * heads; };
+  while (s > tiles::kDecSplitKeysMid && items(s) < tiles::kDecItemsPerWave * waves) s /= 2;
+  while (s > tiles::kDecSplitKeysMin && 2 * items(s) < waves) s /= 2;
   return s;
 }
 
@@ -346,7 +361,7 @@ int device_cu_count() {
 template <class T, int D>
 static hipError_t launch_combine(const fa_decode_args& a, DecodeWs ws, hipStream_t st) {
   hipLaunchKernelGGL((decode_combine_kernel<T, D>), dim3((unsigned)(a.batch * a.num_heads)),
-                     dim3(64), 0, st, a, ws);
+                     dim3(64 * kCombineWaves), 0, st, a, ws);
   return hipGetLastError();
 }
 
@@ -358,10 +373,12 @@ static hipError_t launch_decode_gb(const fa_decode_args& a, DecodeWs ws,
   if (items > 0) {  // max_seq_len == 0: the combine alone writes zeros
     if (use_stream(a)) {
       using SD = DecStream<D>;
-      const int64_t wgs = std::max<int64_t>(
-          1, std::min<int64_t>((items + SD::kWavesPerWG - 1) / SD::kWavesPerWG,
-                               (int64_t)device_cu_count() * SD::kWavesPerCU / SD::kWavesPerWG));
-      DecodeWsS wss{ws.po, ws.plse, ws.split_dev, ws.nsplit, ws.split};
+      // One workgroup per CU as long as there are items for them (few items
+      // are spread over the CUs, each of which streams at its own rate).
+      const int64_t waves = (int64_t)device_cu_count() * SD::kWavesPerCU;
+      const int64_t wgs =
+          std::max<int64_t>(1, std::min<int64_t>(items, waves / SD::kWavesPerWG));
+      DecodeWsS wss{ws.po, ws.plse, ws.split_dev, ws.nsplit, ws.split, (int)waves};
       hipLaunchKernelGGL((decode_stream_kernel<T, SD::D, GB>), dim3((unsigned)wgs),
                          dim3(64 * SD::kWavesPerWG), 0, st, a, wss);
       hipError_t e = hipGetLastError();

@@ -37,8 +37,9 @@
 // prefix-sums these over the batch into LDS, so the grid never holds empty work.
 // split (keys per item) is chosen per call by the launcher from the sizes
 // (max_seq_len); the first wave doubles it when the actual lengths still give
-// every wave kDecItemsPerWave items at twice the split, and workgroup 0
-// records the split it used for the combine kernel.
+// every wave kDecItemsPerWave items at twice the split, or halves it while they
+// give fewer than one item per two waves (and the partials still fit), and
+// workgroup 0 records the split it used for the combine kernel.
 #pragma once
 
 #include "fa355.h"
@@ -49,8 +50,6 @@ namespace fa {
 template <int D_>
 struct DecStream {
   static constexpr int D = D_;
-  static constexpr int kSplitMax = tiles::kDecSplitKeysMax;  // keys per item, largest choice
-  static constexpr int kSplitMin = tiles::kDecSplitKeysMin;  // smallest choice
   static constexpr int kTile = tiles::kDecTileKeys;        // keys per tile
   static constexpr int kMaxBatch = 1024;
   static constexpr int kMaxGroup = 8;  // query heads per item (MFMA columns used)
@@ -80,6 +79,7 @@ struct DecodeWsS {
   int* split_out;  // the split size used (written by workgroup 0)
   int nsplit;      // partials per (sequence, head) the workspace holds at `split`
   int split;       // keys per item chosen by the launcher (a multiple of kTile)
+  int waves;       // waves of a full grid
 };
 
 // Item -> (b, kv head, head group, split, key range) through the batch
@@ -244,13 +244,30 @@ void decode_stream_kernel(fa_decode_args a, DecodeWsS ws) {
   __shared__ int split_sh;
   if (wv == 0) {
     int split = ws.split;
-    int units2 = 0;  // items per head slot at twice the split
-    for (int b0 = 0; b0 < B; b0 += 64) {
-      const int b = b0 + lane;
-      const int len = b < B ? max(0, min(a.seq_lens[b], cap)) : 0;
-      units2 += wave_sum_int((len + 2 * split - 1) / (2 * split));
+    // Items per head slot at a split of n keys.
+    auto units = [&](int n) {
+      int sum = 0;
+      for (int b0 = 0; b0 < B; b0 += 64) {
+        const int b = b0 + lane;
+        const int len = b < B ? max(0, min(a.seq_lens[b], cap)) : 0;
+        sum += wave_total((len + n - 1) / n);
+      }
+      return sum;
+    };
+    if ((int64_t)B * HG * 2 < ws.waves) {
+      // Few sequences: block tables are often as wide as the longest context
+      // the model takes, so the launcher's split can be far too long.
+      int longest = 0;
+      for (int b0 = 0; b0 < B; b0 += 64)
+        longest = max(longest, b0 + lane < B ? max(0, min(a.seq_lens[b0 + lane], cap)) : 0);
+#pragma unroll
+      for (int o = 32; o >= 1; o >>= 1) longest = max(longest, __shfl_xor(longest, o));
+      while (split > tiles::kDecSplitKeysMin &&
+             (longest + split / 2 - 1) / (split / 2) <= ws.nsplit &&  // the partials fit
+             (int64_t)units(split) * HG * 2 < ws.waves)
+        split /= 2;
     }
-    if ((int64_t)units2 * HG >= (int64_t)tiles::kDecItemsPerWave * gridDim.x * W) split *= 2;
+    if ((int64_t)units(2 * split) * HG >= (int64_t)tiles::kDecItemsPerWave * ws.waves) split *= 2;
     if (lane == 0) {
       split_sh = split;
       if (blockIdx.x == 0) *ws.split_out = split;
@@ -263,14 +280,9 @@ void decode_stream_kernel(fa_decode_args a, DecodeWsS ws) {
         const int len = max(0, min(a.seq_lens[b], cap));
         cnt = (len + split - 1) / split;
       }
-      int incl = cnt;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int v = __shfl_up(incl, o);
-        if (lane >= o) incl += v;
-      }
+      const int incl = wave_scan(cnt);
       if (b < B) pfx[b + 1] = base + incl;
-      base += __shfl(incl, 63);
+      base += __builtin_amdgcn_readlane(incl, 63);
     }
     if (lane == 0) pfx[0] = 0;
   }
@@ -282,7 +294,10 @@ void decode_stream_kernel(fa_decode_args a, DecodeWsS ws) {
   // W consecutive items: with HG = W, the W head slots of one split, whose
   // rows share the cache pages and DRAM rows.
   const int total = __builtin_amdgcn_readfirstlane(pfx[B]) * HG;  // uniform: item state stays scalar
-  const int per_wg = (total + gridDim.x * W - 1) / (gridDim.x * W) * W;
+  // Fewer items than waves are spread over the workgroups instead.
+  const int grid = gridDim.x;
+  const int per_wg = total > grid * W ? (total + grid * W - 1) / (grid * W) * W
+                                      : (total + grid - 1) / grid;
   const int I1 = min((int)blockIdx.x * per_wg + per_wg, total);
   const int I0 = blockIdx.x * per_wg + wv;
   if (I0 >= I1) return;

@@ -323,21 +323,6 @@ static int64_t paged_order_grid(int64_t slots, int64_t combos) {
   return (slots + f - 1) / f * f * combos;
 }
 
-// Inclusive prefix sum over the 64 lanes: DPP adds within rows of 16, then
-// row broadcasts (a shuffle goes through LDS, ~10 times the latency).
-__device__ __forceinline__ int wave_scan(int x) {
-  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);  // row_shr:1
-  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);  // row_shr:2
-  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);  // row_shr:4
-  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);  // row_shr:8
-  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, true);  // row_bcast:15
-  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, true);  // row_bcast:31
-  return x;
-}
-__device__ __forceinline__ int wave_total(int x) {
-  return __builtin_amdgcn_readlane(wave_scan(x), 63);
-}
-
 // Finds the sequence owning slot `tile` in the varlen tile space where
 // sequence b has ceil(qlen_b * G / BM) tiles.  Returns b (or -1) and the
 // tile's index from the sequence's last (the one that sees most keys).

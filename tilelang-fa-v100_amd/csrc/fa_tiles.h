@@ -138,7 +138,7 @@ constexpr int kBwdPieceTiles = 16;
 // Persistent waves; work item = a split of keys x one KV head x its query
 // heads (up to 8, the 16x16x32 MFMA columns); 16-key tiles, two in flight
 // per wave.  Keys per split: the largest of kDecSplitKeysMax, /2, /4 ..
-// kDecSplitKeysMin whose item count, estimated from max_seq_len, is at least
+// kDecSplitKeysMid whose item count, estimated from max_seq_len, is at least
 // kDecItemsPerWave per resident wave (long items amortise each item's query
 // load and partial-result store; enough items keep every wave streaming);
 // the kernel doubles it when the actual lengths allow (T2 83%, C4 stays 80%).
@@ -152,8 +152,18 @@ constexpr int kBwdPieceTiles = 16;
 // waves, 512: 2 tiles x 2 waves): 64 x 16k keys at D = 64 76.0%, 64 x 8k at
 // D = 256 83.2%, 64 x 4k at D = 512 79.2% of 8 TB/s, against 63-66% on the
 // chunked kernel below.
+// Below kDecSplitKeysMid, down to kDecSplitKeysMin, while there is less than one
+// item per two waves (a wave walks its item's 16-key tiles serially, two in
+// flight; ~1.3 us each), from max_seq_len on the host and from the actual
+// lengths on the device (block tables are often far wider).  Evidence (us per
+// call, 32 / 8 heads, D = 128, 512-key items / this rule): 4 sequences of
+// 0.5-8k keys 49 / 20, 1 of 4k 45 / 12, 1 of 32k 53 / 30, 32 of 300-700 48 /
+// 21, 16 of 0.5-8k (1100 items of 512) 61 / 57.  Halving until every wave has
+// an item: 24 / 12 / 36 / 26 / 63 (more partials to write and merge); one per
+// four waves: 22 / 12 / 31 / 31 / 57.
 constexpr int kDecSplitKeysMax = 2048;
-constexpr int kDecSplitKeysMin = 512;
+constexpr int kDecSplitKeysMid = 512;
+constexpr int kDecSplitKeysMin = 64;
 constexpr int kDecItemsPerWave = 2;
 constexpr int kDecTileKeys = 16;
 constexpr int kDecTilesInFlight = 2;
