@@ -201,6 +201,29 @@ static void launch_bwd_dq(const fa_bwd_args& a, int mode, float* stats, hipStrea
     hipLaunchKernelGGL((bwd_dq_kernel<T, D, kMaskNone>), grid, block, 0, st, a, stats);
 }
 
+// Waves per workgroup of the dQ-from-dS kernel.  Eight waves share each K tile
+// (half the K traffic of four), but with at most one 8-wave workgroup per CU a
+// causal problem runs as long as its longest one, and below half that a CU
+// has waves to spare: four then, twice as many workgroups (two fit a CU at
+// head_dim 128, one at 256).
+// Measured (fa_bwd per call, us, 8 / 4 waves, same box; 8-wave workgroups in
+// brackets): causal [2, 4096, 8, 256] 455 / 431 (256), [1, 2048, 16, 256] 198 /
+// 180 (128), [1, 2048, 8, 128] 97 / 87 (64), [2, 2048, 16, 128] 173 / 170 (256),
+// [2, 2000, 32/8, 128] 264 / 267 (512), [2, 8192, 8, 256] 1519 / 1557 (512);
+// full [1, 4096, 8, 256] 423 / 399 (128), [1, 4096, 16, 128] 393 / 405 (256).
+static int dq_ds_waves(const fa_bwd_args& a, int mode) {
+  const int64_t wgs8 =
+      ((int64_t)a.seqlen_q + 255) / 256 * a.num_heads * (int64_t)a.batch;
+  const int cus = device_cu_count();
+  return wgs8 <= (mode == kMaskCausal ? cus : cus / 2) ? 4 : 8;
+}
+template <class T, int D, int MODE, int NW>
+static void launch_dq_ds(const fa_bwd_args& a, const uint16_t* ds, hipStream_t st) {
+  const int nqb = ((a.seqlen_q + 31) / 32 + NW - 1) / NW;
+  hipLaunchKernelGGL((bwd_dq_ds_kernel<T, D, MODE, NW>),
+                     dim3((unsigned)nqb * a.num_heads * a.batch), dim3(64 * NW), 0, st, a, ds);
+}
+
 // dS-store path (head_dim 128 / 256): row statistics, dK / dV storing dS,
 // then dQ = dS K (dS includes the scale).
 template <class T, int D>
@@ -217,13 +240,11 @@ static hipError_t launch_bwd_ds(const fa_bwd_args& a, int mode, void* ws, float*
   launch_bwd_main<T, D>(a, mode, stats, ds, part, pieces, st);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
-  constexpr int NW = DqDsShape<D>::NW;
-  const int nqb = ((a.seqlen_q + 31) / 32 + NW - 1) / NW;
-  const dim3 grid((unsigned)nqb * a.num_heads * a.batch), block(64 * NW);
+  const bool four = dq_ds_waves(a, mode) == 4;
   if (mode == kMaskCausal)
-    hipLaunchKernelGGL((bwd_dq_ds_kernel<T, D, kMaskCausal>), grid, block, 0, st, a, ds);
+    four ? launch_dq_ds<T, D, kMaskCausal, 4>(a, ds, st) : launch_dq_ds<T, D, kMaskCausal, 8>(a, ds, st);
   else
-    hipLaunchKernelGGL((bwd_dq_ds_kernel<T, D, kMaskNone>), grid, block, 0, st, a, ds);
+    four ? launch_dq_ds<T, D, kMaskNone, 4>(a, ds, st) : launch_dq_ds<T, D, kMaskNone, 8>(a, ds, st);
   return hipGetLastError();
 }
 

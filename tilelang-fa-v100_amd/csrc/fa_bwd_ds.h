@@ -146,9 +146,9 @@ __global__ __launch_bounds__(256) void bwd_stats_kernel(fa_bwd_args a, float* st
   }
 }
 
-// dQ = Σ_kb dS(qt, kb) K(kb) for head_dim 128 / 256 (dS carries the scale).  Workgroup: 8
-// waves, wave w owns query tile qt = 8 qb + w of one query head; steps run
-// over 32-key blocks.  Per step, wave w copies rows 4w..4w+3 of the K tile
+// dQ = Σ_kb dS(qt, kb) K(kb) for head_dim 128 / 256 (dS carries the scale).  Workgroup: NW
+// waves, wave w owns query tile qt = NW qb + w of one query head; steps run
+// over 32-key blocks.  Per step, wave w copies 32 / NW rows of the K tile
 // and its own 2 KB dS tile HBM -> LDS (buffer DMA: K rows past Sk and dS
 // tiles past the wave's count read as zero), NBUF stages, NBUF - 1 in flight.
 // Products (the layout of bwd_dq_kernel's dQᵀ += Kᵀ dSᵀ):
@@ -159,9 +159,11 @@ __global__ __launch_bounds__(256) void bwd_stats_kernel(fa_bwd_args a, float* st
 // bytes read by lane 16g + 4j + i/4; both operands are read so that lane l
 // gets keys 16kc + 8(l/32) + 4r + j (read r = 0, 1) of column l%32 (d for A,
 // query for B).
-template <int D>
+// NW: 8 waves share a K tile where their workgroups fill the chip; 4 where
+// they do not (dq_ds_waves in fa_bwd.hip).
+template <int D, int NW_>
 struct DqDsShape {
-  static constexpr int NW = 8;                   // (4: C2 71.4 against 68.2 us)
+  static constexpr int NW = NW_;
   static constexpr int RW = 32 / NW;             // K rows each wave copies per step
   static constexpr int ROWB = 2 * D;             // bytes per K row
   static constexpr int RPB = 1024 / ROWB;        // K rows per 1 KB DMA block
@@ -171,20 +173,20 @@ struct DqDsShape {
   // box, dQ kernel: C2 65.8 us against 77.4 (two workgroups per CU with three
   // stages each) and 68.3 (one with six); T1 within noise of both (418-435 us).
   static constexpr int NBUF = 4;
-  static constexpr int WPE = 2;                  // waves per SIMD
+  static constexpr int WPE = 2;                  // waves per SIMD (NW = 4: two workgroups at D = 128)
   static constexpr int KTB = 32 * ROWB;          // K tile: 32 keys
   static constexpr int OFF_S = NBUF * KTB;       // dS stages after the K stages
   static constexpr int SSB = NW * 2048;          // dS stage: one tile per wave
   static constexpr int LDS = OFF_S + NBUF * SSB;
   static_assert((D == 128 || D == 256) && KBPW * RPB * NW == 32, "shape");
-  static_assert(LDS * (WPE / 2) <= 160 * 1024, "LDS");
+  static_assert(LDS <= 160 * 1024, "LDS");
 };
 
-template <class T, int D, int MODE>
-__global__ __launch_bounds__(64 * DqDsShape<D>::NW, DqDsShape<D>::WPE) void bwd_dq_ds_kernel(
+template <class T, int D, int MODE, int NW>
+__global__ __launch_bounds__((64 * NW), (DqDsShape<D, NW>::WPE)) void bwd_dq_ds_kernel(
     fa_bwd_args a, const uint16_t* ds) {
-  using Sh = DqDsShape<D>;
-  constexpr int NW = Sh::NW, ROWB = Sh::ROWB, NBUF = Sh::NBUF, KTB = Sh::KTB, KBPW = Sh::KBPW;
+  using Sh = DqDsShape<D, NW>;
+  constexpr int ROWB = Sh::ROWB, NBUF = Sh::NBUF, KTB = Sh::KTB, KBPW = Sh::KBPW;
   constexpr int OFF_S = Sh::OFF_S, SSB = Sh::SSB;
   __shared__ __attribute__((aligned(16))) char smem[Sh::LDS];
 
@@ -287,7 +289,6 @@ __global__ __launch_bounds__(64 * DqDsShape<D>::NW, DqDsShape<D>::WPE) void bwd_
   // (every wave's part of the K tile landed; the stage of step s - 1 is
   // free), refill that stage with step s + NBUF - 1.
   constexpr int PER_STAGE = KBPW + 2;
-  static_assert(PER_STAGE == 3 || PER_STAGE == 4, "waits below");
   static_assert(NBUF == 4, "stage arithmetic and waits below");
   for (int s = 0; s < NBUF - 1 && s < nsteps; ++s) issue(s, s);
   auto step = [&](int s) {
@@ -298,12 +299,12 @@ __global__ __launch_bounds__(64 * DqDsShape<D>::NW, DqDsShape<D>::WPE) void bwd_
   // All but the last two steps leave two stages in flight: one fixed wait.
   int s = 0;
   for (; s + 2 < nsteps; ++s) {
-    __builtin_amdgcn_s_waitcnt(PER_STAGE == 3 ? 0x0F76 : 0x0F78);  // vmcnt(2 PER_STAGE)
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PER_STAGE) : "memory");
     step(s);
   }
   for (; s < nsteps; ++s) {
     if (s + 1 < nsteps)
-      __builtin_amdgcn_s_waitcnt(PER_STAGE == 3 ? 0x0F73 : 0x0F74);  // vmcnt(PER_STAGE)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER_STAGE) : "memory");
     else
       wait_vmem();
     step(s);
