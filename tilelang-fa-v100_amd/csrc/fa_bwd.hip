@@ -48,18 +48,28 @@ static size_t stats_bytes(const fa_bwd_args& a) {
 static size_t ds_offset(const fa_bwd_args& a) { return (stats_bytes(a) + 255) & ~(size_t)255; }
 
 // Bytes of dS tiles for the dS-store path, or 0 where it does not apply:
-// head_dim 128 / 256, causal or full attention, below tiles::kBwdDsMaxBytes.
-static size_t ds_bytes(const fa_bwd_args& a) {
-  const int mode = mask_mode(a);
-  if ((a.head_dim != 128 && a.head_dim != 256) || mode == kMaskBand || a.seqlen_q <= 0 ||
-      a.seqlen_k <= 0)
-    return 0;
-  const DsTiles L = mode == kMaskCausal ? ds_tiles<kMaskCausal>(a.seqlen_q, a.seqlen_k)
-                                        : ds_tiles<kMaskNone>(a.seqlen_q, a.seqlen_k);
+// head_dim 128 / 256, below tiles::kBwdDsMaxBytes.
+template <int MODE>
+static size_t ds_bytes_of(const fa_bwd_args& a) {
+  if ((a.head_dim != 128 && a.head_dim != 256) || a.seqlen_q <= 0 || a.seqlen_k <= 0) return 0;
+  const Band band = make_band(a);
+  const DsTiles<MODE> L = ds_tiles<MODE>(a.seqlen_q, a.seqlen_k, band.wl, band.wr);
   const size_t bytes = 2048 * (size_t)a.batch * a.num_heads * (size_t)L.per_head();
   // Strictly below the cap: a wave's dS reads go through one buffer resource
   // of count(qt) * 2 KB bytes (a 32-bit size), and count(qt) <= per_head.
   return bytes < tiles::kBwdDsMaxBytes ? bytes : 0;
+}
+// Causal and full attention: part of bwd_workspace_bytes.
+static size_t ds_bytes(const fa_bwd_args& a) {
+  const int mode = mask_mode(a);
+  return mode == kMaskCausal ? ds_bytes_of<kMaskCausal>(a)
+                             : (mode == kMaskNone ? ds_bytes_of<kMaskNone>(a) : 0);
+}
+// Window bands: part of bwd_preferred_workspace_bytes only.
+static size_t band_ds_bytes(const fa_bwd_args& a) {
+  return mask_mode(a) == kMaskBand && (int64_t)a.seqlen_q + a.seqlen_k < (1 << 29)
+             ? ds_bytes_of<kMaskBand>(a)
+             : 0;
 }
 
 size_t bwd_min_workspace_bytes(const fa_bwd_args& a) { return stats_bytes(a); }
@@ -139,6 +149,7 @@ static size_t part_bytes(const fa_bwd_args& a, int pieces) {
 static size_t part_offset(const fa_bwd_args& a) { return (bwd_workspace_bytes(a) + 255) & ~(size_t)255; }
 
 size_t bwd_preferred_workspace_bytes(const fa_bwd_args& a) {
+  if (const size_t ds = band_ds_bytes(a)) return ds_offset(a) + ds;
   const int pieces = bwd_pieces(a);
   return pieces > 1 ? part_offset(a) + part_bytes(a, pieces) : bwd_workspace_bytes(a);
 }
@@ -166,10 +177,12 @@ template <class T, int D, int MODE>
 static void launch_bwd_main(const fa_bwd_args& a, const float* stats, uint16_t* ds, float* part,
                             int pieces, hipStream_t st) {
   if (a.seqlen_k == 0) return;  // no keys: dK / dV are empty
-  constexpr bool kDs = D >= 128 && MODE != kMaskBand;
+  constexpr bool kDs = D >= 128;
   constexpr bool kSplit = MODE != kMaskBand;
   if constexpr (kDs) {
-    if (ds && pieces > 1) return launch_main<T, D, MODE, true, true>(a, stats, ds, part, pieces, st);
+    if constexpr (kSplit)
+      if (ds && pieces > 1)
+        return launch_main<T, D, MODE, true, true>(a, stats, ds, part, pieces, st);
     if (ds) return launch_main<T, D, MODE, true, false>(a, stats, ds, nullptr, 1, st);
   } else if constexpr (kSplit) {
     if (pieces > 1) return launch_main<T, D, MODE, false, true>(a, stats, nullptr, part, pieces, st);
@@ -241,7 +254,9 @@ static hipError_t launch_bwd_ds(const fa_bwd_args& a, int mode, void* ws, float*
   e = hipGetLastError();
   if (e != hipSuccess) return e;
   const bool four = dq_ds_waves(a, mode) == 4;
-  if (mode == kMaskCausal)
+  if (mode == kMaskBand)
+    four ? launch_dq_ds<T, D, kMaskBand, 4>(a, ds, st) : launch_dq_ds<T, D, kMaskBand, 8>(a, ds, st);
+  else if (mode == kMaskCausal)
     four ? launch_dq_ds<T, D, kMaskCausal, 4>(a, ds, st) : launch_dq_ds<T, D, kMaskCausal, 8>(a, ds, st);
   else
     four ? launch_dq_ds<T, D, kMaskNone, 4>(a, ds, st) : launch_dq_ds<T, D, kMaskNone, 8>(a, ds, st);
@@ -262,7 +277,9 @@ static hipError_t launch_bwd_d(const fa_bwd_args& a, void* ws, size_t ws_bytes, 
                     ? reinterpret_cast<float*>(static_cast<char*>(ws) + part_offset(a))
                     : nullptr;
   if constexpr (D >= 128) {
-    if (ds_bytes(a) && ws_bytes >= bwd_workspace_bytes(a))
+    const size_t band_ds = band_ds_bytes(a);
+    if (band_ds ? ws_bytes >= ds_offset(a) + band_ds
+                : ds_bytes(a) && ws_bytes >= bwd_workspace_bytes(a))
       return launch_bwd_ds<T, D>(a, mode, ws, part, pieces, st);
   }
   float* stats = static_cast<float*>(ws);  // [B*H][2][Sq]

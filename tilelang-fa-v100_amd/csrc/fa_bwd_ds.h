@@ -1,5 +1,5 @@
 // dQ of the dense attention backward from stored dS tiles (head_dim 128 and
-// 256, causal or full attention).
+// 256).
 //
 // The key-stationary dK / dV kernel (fa_bwd_mfma.h) forms dS = P (dP −
 // rowdot)·scale for every (query tile, key block) pair it visits.  With its
@@ -14,8 +14,9 @@
 //
 // Tile layout: query head bh = b·H + h, query tile qt (rows 32qt..32qt+31)
 // and key block kb (keys 32kb..32kb+31) with kb < count(qt) own the 2 KB at
-//   ds + 2048 · (bh · per_head + prefix(qt) + kb),
-// prefix(qt) = Σ_{t<qt} count(t).  A tile is two 1 KB blocks kq = 0, 1; lane
+//   ds + 2048 · (bh · per_head + prefix(qt) + kb - lo(qt)),
+// prefix(qt) = Σ_{t<qt} count(t) and lo = 0 except for window bands (DsTiles).
+// A tile is two 1 KB blocks kq = 0, 1; lane
 // (key, half) of the writing wave packs dS of query rows 16kq + 8(x/4) +
 // 4 half + x%4, x = 0..7, as its chunk kq and stores it as 16-byte row
 // 16(2(key/16) + (key/8)%2) + 8 half + 4(((key/4)%2) ^ kq) + key%4 of block kq:
@@ -56,11 +57,17 @@ __device__ __forceinline__ void buffer_lds16_stream2(u32x4 rsrc, uint32_t voff, 
       : "memory");
 }
 
-// Per-head tile counts of the dS workspace.  count(t): key blocks a query
-// tile reaches; causal (keys j <= i + Sk - Sq): kb <= t + floor((31 + Sk -
-// Sq) / 32), clipped to [0, nk]; full attention: every block.
+__host__ __device__ inline int floor_div32(int x) { return x >= 0 ? x / 32 : -((31 - x) / 32); }
+
+// Per-head tile counts of the dS workspace.  Query tile t reaches the key
+// blocks lo(t) .. lo(t) + count(t) - 1, whose tiles follow one another from
+// prefix(t) on.  Causal (keys j <= i + Sk - Sq): blocks below t + floor((31 +
+// Sk - Sq) / 32) + 1, clipped to [0, nk]; full attention: every block; their
+// rows of tiles are packed.
+template <int MODE>
 struct DsTiles {
   int nq, nk, c1;
+  __host__ __device__ int lo(int) const { return 0; }
   __host__ __device__ int count(int t) const { return min(max(t + c1, 0), nk); }
   // Σ_{t<n} count(t): zero below t0 = -c1, t + c1 up to t = nk - c1, then nk.
   __host__ __device__ int64_t prefix(int n) const {
@@ -71,16 +78,37 @@ struct DsTiles {
     return ramp + (int64_t)(n - t1) * nk;
   }
   __host__ __device__ int64_t per_head() const { return prefix(nq); }
+  // Tiles from block kb of query tile t to block kb of tile t + 1.
+  __host__ __device__ int step(int t) const { return count(t); }
+};
+// Window band (keys i + off - wl <= j <= i + off + wr, -1 unbounded): blocks
+// max(t + cl, 0) .. min(t + c1, nk) - 1 with cl = floor((off - wl) / 32) and c1 =
+// floor((31 + off + wr) / 32) + 1; every query tile has room for `width`
+// blocks, the most a tile reaches.
+template <>
+struct DsTiles<kMaskBand> {
+  int nq, nk, c1, cl, width;
+  __host__ __device__ int lo(int t) const { return min(max(t + cl, 0), nk); }
+  __host__ __device__ int count(int t) const { return max(min(t + c1, nk) - lo(t), 0); }
+  __host__ __device__ int64_t prefix(int n) const { return (int64_t)n * width; }
+  __host__ __device__ int64_t per_head() const { return prefix(nq); }
+  __host__ __device__ int step(int t) const { return width - (lo(t + 1) - lo(t)); }
 };
 
-__host__ __device__ inline int floor_div32(int x) { return x >= 0 ? x / 32 : -((31 - x) / 32); }
-
 template <int MODE>
-__host__ __device__ inline DsTiles ds_tiles(int sq, int sk) {
-  static_assert(MODE == kMaskCausal || MODE == kMaskNone, "dS tiles: causal or full");
+__host__ __device__ inline DsTiles<MODE> ds_tiles(int sq, int sk, int wl = -1, int wr = -1) {
   const int nq = (sq + 31) / 32, nk = (sk + 31) / 32;
-  const int c1 = MODE == kMaskCausal ? floor_div32(31 + sk - sq) + 1 : nk;
-  return DsTiles{nq, nk, c1};
+  if constexpr (MODE == kMaskBand) {
+    // Bounds clamped to the lengths keep the sums in 32 bits; a bound at or past
+    // the other end hides nothing.
+    const int far = sq + sk, off = sk - sq;
+    const int c1 = wr < 0 ? nk + nq : floor_div32(31 + off + min(wr, far)) + 1;
+    const int cl = wl < 0 ? -nk - nq : floor_div32(off - min(wl, far));
+    return DsTiles<MODE>{nq, nk, c1, cl, max(min(nk, c1 - cl), 0)};
+  } else {
+    const int c1 = MODE == kMaskCausal ? floor_div32(31 + sk - sq) + 1 : nk;
+    return DsTiles<MODE>{nq, nk, c1};
+  }
 }
 
 // Row statistics [B*H][2][Sq] fp32 for the dK / dV kernel: LSE·log2(e) (+inf
@@ -191,18 +219,23 @@ __global__ __launch_bounds__((64 * NW), (DqDsShape<D, NW>::WPE)) void bwd_dq_ds_
   __shared__ __attribute__((aligned(16))) char smem[Sh::LDS];
 
   const int Sq = a.seqlen_q, Sk = a.seqlen_k, H = a.num_heads;
-  const DsTiles L = ds_tiles<MODE>(Sq, Sk);
+  const Band band = mode_band<MODE>(a);
+  const DsTiles<MODE> L = ds_tiles<MODE>(Sq, Sk, band.wl, band.wr);
   const int nqb = (L.nq + NW - 1) / NW;
   const TileHead th = xcd_tile_order(blockIdx.x, nqb, a.batch * H);
   const int bh = th.bh, h = bh % H, b = bh / H;
   const int hk = h / (H / a.num_heads_k);
-  // Causal: the longest query tiles (largest index) first.
+  // Causal: the longest query tiles (largest index) first.  (A band's are
+  // alike.)
   const int qb = MODE == kMaskCausal ? nqb - 1 - th.rank : th.rank;
   const int lane = threadIdx.x & 63, wave = wave_id();
   const int lr = lane & 31, lh = lane >> 5;
   const int qt = NW * qb + wave;
   const int cnt = qt < L.nq ? L.count(qt) : 0;
-  const int nsteps = L.count(min(NW * qb + NW - 1, L.nq - 1));
+  // Key blocks s0 .. s0 + nsteps - 1 of the workgroup, [w0, w0 + cnt) of the wave.
+  const int qt_last = min(NW * qb + NW - 1, L.nq - 1);
+  const int s0 = L.lo(NW * qb), w0 = L.lo(min(qt, L.nq));
+  const int nsteps = max(L.lo(qt_last) + L.count(qt_last) - s0, 0);
 
   // K rows 32s + 4w + rr, rr = RPB i + lane / CPR in block i, stored chunk
   // lane % CPR (logical chunk (lane % CPR) ^ swz(row), the swizzle acting on
@@ -223,10 +256,10 @@ __global__ __launch_bounds__((64 * NW), (DqDsShape<D, NW>::WPE)) void bwd_dq_ds_
   // at the wave's first row of that step and carried: one 64-bit add per
   // step; num_records covers RW rows except where they run past Sk.
   const uint32_t k_full = span_bytes(Sh::RW, a.k_stride[1], D);
-  u32x4 rk = rsrc_words(kg + (int64_t)(Sh::RW * wave) * a.k_stride[1], k_full);
+  u32x4 rk = rsrc_words(kg + (int64_t)(32 * s0 + Sh::RW * wave) * a.k_stride[1], k_full);
   const uint64_t k_step = 2ull * 32 * (uint64_t)a.k_stride[1];
   auto issue = [&](int s, int stage) {
-    const int nb = 32 * s + Sh::RW * wave;
+    const int nb = 32 * (s0 + s) + Sh::RW * wave;
     u32x4 r = rk;
     if (nb + Sh::RW > Sk)
       r[2] = __builtin_amdgcn_readfirstlane(
@@ -237,7 +270,9 @@ __global__ __launch_bounds__((64 * NW), (DqDsShape<D, NW>::WPE)) void bwd_dq_ds_
     const uint64_t p = (((uint64_t)rk[1]) << 32 | rk[0]) + k_step;
     rk[0] = (uint32_t)p;
     rk[1] = (uint32_t)(p >> 32);
-    buffer_lds16_stream2(rs, (uint32_t)s * 2048u + 16u * lane, smem + OFF_S + stage * SSB + wave * 2048);
+    // (A block before the wave's first wraps to an offset past its range, like
+    // one after its last: it reads as zero.)
+    buffer_lds16_stream2(rs, (uint32_t)(s0 + s - w0) * 2048u + 16u * lane, smem + OFF_S + stage * SSB + wave * 2048);
   };
 
   // Transpose-read offsets.  A, read r, d tile dt: row 8(lane/32) + 4r +
@@ -294,7 +329,7 @@ __global__ __launch_bounds__((64 * NW), (DqDsShape<D, NW>::WPE)) void bwd_dq_ds_
   auto step = [&](int s) {
     __syncthreads();
     if (s + NBUF - 1 < nsteps) issue(s + NBUF - 1, (s + NBUF - 1) & (NBUF - 1));
-    if (s < cnt) compute(s & (NBUF - 1));
+    if ((unsigned)(s0 + s - w0) < (unsigned)cnt) compute(s & (NBUF - 1));
   };
   // All but the last two steps leave two stages in flight: one fixed wait.
   int s = 0;

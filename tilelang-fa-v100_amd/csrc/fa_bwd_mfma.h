@@ -54,7 +54,7 @@ struct TrOps {
 
 // MODE (MaskMode): full attention, causal, or a window band from the arguments.
 // DS: also store every computed 32 x 32 dS block to `ds` (tile layout of
-// fa_bwd_ds.h; causal or full attention) for bwd_dq_ds_kernel.
+// fa_bwd_ds.h) for bwd_dq_ds_kernel.
 // SPLIT: the workgroup's query tiles (G heads x the tiles that see its keys)
 // are cut into nsplit consecutive pieces, one workgroup each; every piece
 // writes its fp32 dK / dV to `part` in accumulator order and
@@ -234,13 +234,13 @@ void bwd_main_mfma_kernel(fa_bwd_args a, const float* stats, uint16_t* ds, float
   const float* s_i = s_top + 2 * h0 * Sq - r0 * S::BQ;
   // DS: the dS tile of the tile `step` computes next (same sweep order as
   // the issue side), stepped back by count(it) tiles per query tile.
-  static_assert(!DS || MODE != kMaskBand, "dS tiles: causal or full attention");
-  DsTiles dsl{1, 1, 1};
+  DsTiles<MODE> dsl{};
   uint16_t* ds_top = nullptr;
   if constexpr (DS) {
-    dsl = ds_tiles<(MODE == kMaskCausal ? kMaskCausal : kMaskNone)>(Sq, Sk);
-    ds_top = ds + 1024 * ((int64_t)(b * H + hk * G) * dsl.per_head() +
-                          dsl.prefix(max(it1, 1) - 1) + kvw / 32);
+    dsl = ds_tiles<MODE>(Sq, Sk, band.wl, band.wr);
+    const int top = max(it1, 1) - 1;
+    ds_top = ds + 1024 * ((int64_t)(b * H + hk * G) * dsl.per_head() + dsl.prefix(top) + kvw / 32 -
+                          dsl.lo(top));
   }
   uint16_t* ds_c = ds_top;
   if constexpr (DS && SPLIT) {
@@ -309,16 +309,27 @@ void bwd_main_mfma_kernel(fa_bwd_args a, const float* stats, uint16_t* ds, float
   // offsets of its Q, dO and statistics tiles.  Returns whether the wave
   // stored a dS tile (DS: two global stores, the wave's newest memory
   // operations).
-  // Causal / full attention: tile `it` (rows i0 .. i0 + BQ - 1) is active
-  // for this wave iff i0 >= act_lo (some row sees key kvw: kvw <= i0 + BQ - 1
-  // + off) and needs no mask iff unm_lo <= i0 <= unm_hi (every row sees the
-  // wave's last key, the wave's 32 keys and the tile's rows all exist): two
-  // comparisons per tile instead of the band tests.
+  // Tile `it` (rows i0 .. i0 + BQ - 1) is active for this wave iff i0 >= act_lo
+  // (some row sees key kvw: kvw <= i0 + BQ - 1 + off + wr) and, in a band, i0 <=
+  // act_hi (some row sees key kvw + 31: kvw + 31 >= i0 + off - wl), and needs no
+  // mask iff unm_lo <= i0 <= unm_hi (every row sees the wave's first and last
+  // key, the wave's 32 keys and the tile's rows all exist): two comparisons
+  // per tile each instead of the band tests.
   const int wkv_last = min(kvw + 31, Sk - 1);
   constexpr int kNever = 0x7fffffff, kAlways = -0x7fffffff;
   const int act_lo = kvw >= Sk ? kNever : MODE == kMaskCausal ? kvw - (S::BQ - 1) - off : kAlways;
   const int unm_lo = kvw + 32 > Sk ? kNever : MODE == kMaskCausal ? wkv_last - off : kAlways;
   const int unm_hi = Sq - S::BQ;
+  int b_act_lo = act_lo, b_act_hi = kNever, b_unm_lo = unm_lo, b_unm_hi = unm_hi;
+  if constexpr (MODE == kMaskBand) {
+    // (Bounds at or past the lengths hide nothing; clamped, the sums stay in
+    // 32 bits.)
+    const int far = Sq + Sk, wr = min(band.wr, far), wl = min(band.wl, far);
+    if (kvw < Sk && wr >= 0) b_act_lo = kvw - (S::BQ - 1) - off - wr;
+    if (wl >= 0) b_act_hi = kvw + 31 - off + wl;
+    if (kvw + 32 <= Sk && wr >= 0) b_unm_lo = wkv_last - off - wr;
+    if (wl >= 0) b_unm_hi = min(unm_hi, kvw - (S::BQ - 1) - off + wl);
+  }
   auto step = [&](int it, int qo, int oo, int so) -> bool {
     const char* qb = smem + qo;
     const char* ob = smem + oo;
@@ -328,11 +339,9 @@ void bwd_main_mfma_kernel(fa_bwd_args a, const float* stats, uint16_t* ds, float
     // every XOR result out of the loop into a register of its own.
     asm volatile("" : "+v"(rb), "+v"(tb0), "+v"(tb1), "+v"(rbk));
     const int i0 = it * S::BQ;
-    // Causal: the wave skips tiles none of its keys see.  A general band
-    // runs such tiles through the masked path instead (P = 0): its two-sided
-    // test makes the register allocator spill heavily, and they are at most
-    // BKV / BQ tiles per workgroup.
-    const bool active = MODE == kMaskBand ? kvw < Sk : i0 >= act_lo;
+    // The wave skips tiles none of its keys see.
+    const bool active =
+        MODE == kMaskBand ? i0 >= b_act_lo && i0 <= b_act_hi : i0 >= act_lo;
     if (!active) return false;
     f32x16 s, dp;
 #pragma unroll
@@ -350,9 +359,7 @@ void bwd_main_mfma_kernel(fa_bwd_args a, const float* stats, uint16_t* ds, float
     sched_pipeline<D / 16, 3, 2, 2>();
 
     const bool need_mask =
-        MODE == kMaskBand
-            ? !band.all(i0, i0 + S::BQ - 1, kvw, wkv_last) || (kvw + 32 > Sk) || (i0 + S::BQ > Sq)
-            : i0 < unm_lo || i0 > unm_hi;
+        MODE == kMaskBand ? i0 < b_unm_lo || i0 > b_unm_hi : i0 < unm_lo || i0 > unm_hi;
     // P = exp2(S·scale·log2e − lse2), dS = P (dP·scale − scale·rowdot).  The
     // statistics hold scale·rowdot, so the scale costs nothing.  Element (g, r)
     // is query i0 + 8g + 4lh + r; on masked tiles it sees the lane's key iff
@@ -445,7 +452,7 @@ void bwd_main_mfma_kernel(fa_bwd_args a, const float* stats, uint16_t* ds, float
       ++h_rel;
       if constexpr (DS) ds_c = ds_top + 1024 * h_rel * dsl.per_head();
     } else if constexpr (DS) {
-      ds_c -= 1024 * dsl.count(it);
+      ds_c -= 1024 * dsl.step(it);
     }
   };
   int ih = h0, ii = it1 - 1 - r0;  // tile to issue next

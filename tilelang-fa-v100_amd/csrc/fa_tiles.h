@@ -101,9 +101,14 @@ constexpr int kBwdQueryRows = 32;
 // cycles per instruction, a floor of ~1.17 ms for T1's backward.
 
 // ---- backward: dQ from stored dS tiles (fa_bwd_ds.h), head_dim 128 / 256,
-// causal or full attention, while the tiles (2 bytes per visible (query, key)
-// pair, 2.15 GB at T1) stay within this many bytes; larger problems recompute
-// S and dP in bwd_dq_kernel.
+// while the tiles (2 bytes per visible (query, key) pair, 2.15 GB at T1; a
+// window band takes its width in whole 32-key blocks per 32 rows) stay within
+// this many bytes; larger problems recompute S and dP in bwd_dq_kernel.
+// Evidence for bands (fa_bwd per call, us, recompute / dS, same box, both with
+// the dK / dV kernel skipping the tiles outside a wave's band): causal,
+// [2, 4096, 16, 128] window 1024 287 / 236, window 256 175 / 143, [2, 8192, 8,
+// 128] window 4096 777 / 691, [2, 4096, 8, 256] window 1024 276 / 227, [1, 1024,
+// 8, 128] window 200 60 / 48.
 constexpr size_t kBwdDsMaxBytes = size_t(4) << 30;
 
 // ---- backward dK / dV kernel, head_dim 64 (fa_bwd_mfma.h): 128 keys per
