@@ -1,4 +1,5 @@
-"""Builds libfa355.so (the gfx950 HIP kernels + C ABI) in-tree with hipcc.
+"""Builds libfa355.so (the gfx950 HIP kernels + C ABI) in-tree with hipcc, and
+_fa_torch.so (the Python calls' native marshalling) with the host compiler.
 
 Usage: python tilelang-fa-v100_amd/build.py [-v]
 
@@ -22,6 +23,7 @@ CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(REPO, "include")
 BUILD = os.path.join(REPO, "_build")
 LIB = os.path.join(HERE, "tilelang_fa_v100", "libfa355.so")
+EXT = os.path.join(HERE, "tilelang_fa_v100", "_fa_torch.so")
 
 SOURCES = ["fa_fwd.hip", "fa_bwd.hip", "fa_decode.hip", "fa_cache.hip", "fa_scratch.hip",
            "fa_capi.cpp"]
@@ -78,6 +80,26 @@ def _run(cmd: list[str], verbose: bool) -> None:
         print(res.stdout + res.stderr, flush=True)
 
 
+def _ext_command() -> list[str]:
+    """Host-only C++ against torch's headers; it gets the library's entry
+    points as addresses, so it links neither libfa355.so nor the HIP runtime."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    cxx = os.environ.get("CXX") or shutil.which("g++") or shutil.which("c++")
+    if not cxx:
+        raise RuntimeError("no host C++ compiler found (set CXX)")
+    inc = [f"-I{p}" for p in (*cpp_extension.include_paths(), sysconfig.get_paths()["include"],
+                              INCLUDE)]
+    libs = [f"-L{p}" for p in cpp_extension.library_paths()]
+    return [cxx, "-O2", "-std=c++17", "-fPIC", "-shared",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *inc,
+            os.path.join(CSRC, "fa_torch.cpp"), "-o", EXT + ".tmp", *libs,
+            "-ltorch_python", "-ltorch_cpu", "-lc10"]
+
+
 def build(verbose: bool = False, extra_flags: list[str] | None = None) -> str:
     """Compiles every source and links the shared library; returns its path."""
     os.makedirs(BUILD, exist_ok=True)
@@ -90,12 +112,14 @@ def build(verbose: bool = False, extra_flags: list[str] | None = None) -> str:
         objs.append(obj)
         cmds.append([cc, *flags, *SOURCE_FLAGS.get(src, []), "-x", "hip", "-c",
                      os.path.join(CSRC, src), "-o", obj])
+    cmds.append(_ext_command())
     with cf.ThreadPoolExecutor(max_workers=min(len(cmds), os.cpu_count() or 4)) as ex:
         for fut in [ex.submit(_run, c, verbose) for c in cmds]:
             fut.result()
     tmp = LIB + ".tmp"
     _run([cc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs], verbose)
     os.replace(tmp, LIB)
+    os.replace(EXT + ".tmp", EXT)
     return LIB
 
 

@@ -13,7 +13,7 @@ import ctypes
 
 import torch
 
-from . import _lib
+from . import _lib, _native
 from ._checks import require_cuda, require_half, require_same, rows_ready, strides
 
 
@@ -25,6 +25,8 @@ def reshape_and_cache(key, value, key_cache, value_cache, slot_mapping):
     or one at or beyond num_pages * page_size leaves the caches untouched.
     The caches are modified in place; nothing is returned.
     """
+    if _native.cache_write(key, value, key_cache, value_cache, slot_mapping) is not None:
+        return
     for name, t in (("key", key), ("value", value), ("key_cache", key_cache),
                     ("value_cache", value_cache)):
         require_half(t, name)

@@ -18,7 +18,7 @@ import math
 
 import torch
 
-from . import _lib
+from . import _lib, _native
 from ._checks import (PAGED_HEAD_DIMS, as_int32, require_cuda, require_half, require_same,
                       rows_ready, strides)
 
@@ -87,6 +87,11 @@ def decode_forward(q, k_cache, v_cache, block_table, seq_lens,
                    block_size=16, num_kv_heads=None, softmax_scale=None,
                    return_lse=False):
     """Paged decode forward; see the module docstring."""
+    if not return_lse:
+        out = _native.decode(q, k_cache, v_cache, block_table, seq_lens, block_size, num_kv_heads,
+                             softmax_scale)
+        if out is not None:
+            return out
     a, out, lse, keep = _decode_args(q, k_cache, v_cache, block_table, seq_lens, block_size,
                                      num_kv_heads, softmax_scale, return_lse)
     lib = _lib.load()

@@ -136,6 +136,21 @@ def set_backward_workspace_limit(nbytes):
     _workspace_limit = nbytes
 
 
+def _cached_unused(device) -> int:
+    """Bytes torch's allocator holds on `device` without a tensor in them.
+
+    From the nested statistics where the allocator runs: memory_reserved()
+    and memory_allocated() each flatten and sort all of them first, ~37 us a
+    call, 0.07 ms of a backward whose GPU work waits for it.
+    """
+    if isinstance(device, torch.device) and device.index is not None and \
+            torch.cuda.is_initialized():
+        stats = torch._C._cuda_memoryStats(device.index)
+        return max(stats["reserved_bytes"]["all"]["current"]
+                   - stats["allocated_bytes"]["all"]["current"], 0)
+    return max(torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device), 0)
+
+
 def workspace_limit(device, want=None) -> int:
     """Bytes the backward's workspace may take on `device` right now.
 
@@ -152,7 +167,7 @@ def workspace_limit(device, want=None) -> int:
             return max(int(env), 0)
         except ValueError:
             raise ValueError(f"{WORKSPACE_LIMIT_ENV} must be a byte count, got {env!r}") from None
-    cached = max(torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device), 0)
+    cached = _cached_unused(device)
     if want is not None and want <= cached:
         return cached
     free, _ = torch.cuda.mem_get_info(device)

@@ -186,6 +186,7 @@ def call_on(device: torch.device, fn):
     (a few microseconds per call) is skipped.
     """
     if device.index == torch.cuda.current_device():
-        return fn(torch.cuda.current_stream().cuda_stream)
+        # (torch.cuda.current_stream() builds a Stream object: ~2.5 us.)
+        return fn(torch._C._cuda_getCurrentRawStream(device.index))
     with torch.cuda.device(device):
         return fn(torch.cuda.current_stream(device).cuda_stream)

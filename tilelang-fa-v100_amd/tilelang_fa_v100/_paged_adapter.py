@@ -22,7 +22,7 @@ import math
 
 import torch
 
-from . import _lib
+from . import _lib, _native
 from ._checks import (PAGED_HEAD_DIMS, as_int32, require_cuda, require_half, require_same,
                       rows_ready, strides)
 
@@ -31,6 +31,12 @@ def paged_forward(q, k_cache, v_cache, block_table, seq_lens,
                   query_start_loc, prefix_kv_lens, out=None,
                   block_size=16, num_kv_heads=None, softmax_scale=None,
                   causal=True, sliding_window_q=-1, sliding_window_k=-1):
+    if out is None:
+        done = _native.paged_forward(q, k_cache, v_cache, block_table, seq_lens, query_start_loc,
+                                     prefix_kv_lens, block_size, num_kv_heads, softmax_scale,
+                                     causal, sliding_window_q, sliding_window_k)
+        if done is not None:
+            return done
     return paged_forward_splits(q, k_cache, v_cache, block_table, seq_lens, query_start_loc,
                                 prefix_kv_lens, out, block_size, num_kv_heads, softmax_scale,
                                 causal, sliding_window_q, sliding_window_k)

@@ -23,7 +23,7 @@ from __future__ import annotations
 
 import torch
 
-from . import _dense
+from . import _dense, _native
 from ._checks import require_cuda, require_half, require_same
 from ._decode_adapter import decode_forward as _decode_forward
 from ._paged_adapter import paged_forward as _paged_forward
@@ -41,21 +41,25 @@ class FlashAttnTileLangVFunc(torch.autograd.Function):
             raise NotImplementedError("alibi not supported")
         if softcap != 0.0:
             raise NotImplementedError("softcap not supported")
-        for name, t in (("q", q), ("k", k), ("v", v)):
-            require_half(t, name)
-        require_same({"q": q, "k": k, "v": v}, "dtype")
-        shapes = _dense.check_shapes(q, k, v)
-        for name, t in (("q", q), ("k", k), ("v", v)):
-            require_cuda(t, name)
-        require_same({"q": q, "k": k, "v": v}, "device")
-        scale = softmax_scale if softmax_scale is not None else q.shape[-1] ** -0.5
-        window = _dense.window_bounds(window_size)
         # Without gradients and without a requested LSE (inference) the kernel
         # skips the LSE store, as the reference's tilelang_forward does
         # (_kernels_forward.py:176-185).
         with_lse = bool(return_softmax) or any(ctx.needs_input_grad[:3])
-        out, lse = _dense.forward(q, k, v, scale, causal, window, shapes=shapes,
+        scale, window = softmax_scale, window_size
+        done = _native.dense_forward(q, k, v, scale, causal, window, with_lse)
+        if done is None:
+            for name, t in (("q", q), ("k", k), ("v", v)):
+                require_half(t, name)
+            require_same({"q": q, "k": k, "v": v}, "dtype")
+            shapes = _dense.check_shapes(q, k, v)
+            for name, t in (("q", q), ("k", k), ("v", v)):
+                require_cuda(t, name)
+            require_same({"q": q, "k": k, "v": v}, "device")
+            scale = softmax_scale if softmax_scale is not None else q.shape[-1] ** -0.5
+            window = _dense.window_bounds(window_size)
+            done = _dense.forward(q, k, v, scale, causal, window, shapes=shapes,
                                   with_lse=with_lse)
+        out, lse = done
         ctx.save_for_backward(q, k, v, out, lse)
         ctx.causal = bool(causal)
         ctx.window = window
