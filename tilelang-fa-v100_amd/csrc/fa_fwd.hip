@@ -326,16 +326,19 @@ static int64_t paged_order_grid(int64_t slots, int64_t combos) {
 // Finds the sequence owning slot `tile` in the varlen tile space where
 // sequence b has ceil(qlen_b * G / BM) tiles.  Returns b (or -1) and the
 // tile's index from the sequence's last (the one that sees most keys).
-// Up to 64 sequences, one per lane of wave 0, in one of two orders; u_b is the
+// Up to 64 sequences, one per lane of wave 0, in one of three orders; u_b is the
 // history in units of a tile's rows, u_b + i + 1 the reach of tile i:
-//  * grids of few rounds (tiles x combos up to kPagedTileOrderMax): all tiles by
-//    decreasing reach, ties by sequence.  Sequence b has n_b(K) = clamp(u_b +
-//    ntiles_b - K, 0, ntiles_b) tiles of reach above K;
-//  * larger grids: sequences by decreasing history (the tiles of one share its
-//    K / V in the L2, and the tail is a small part), n_b(K) = all or none.
-// Either way a binary search for the smallest K with at most `tile` tiles above
-// it, and the slot's rank among those at K, name the tile.  More sequences are
-// scanned in their own order, 64 at a time.
+//  * grids that start at once (tiles x combos up to kPagedOneRound), and larger
+//    ones than two rounds without histories to tell sequences apart: by sequence
+//    (the search below costs ~0.6 us a workgroup);
+//  * grids of two rounds (up to kPagedTileOrderMax): all tiles by decreasing
+//    reach, ties by sequence.  Sequence b has n_b(K) = clamp(u_b + ntiles_b - K,
+//    0, ntiles_b) tiles of reach above K;
+//  * larger grids: sequences by the reach of their last tile, longest first (the
+//    tiles of one share its K / V in the L2), n_b(K) = all or none.
+// For the last two a binary search for the smallest K with at most `tile` tiles
+// above it, and the slot's rank among those at K, name the tile.  More
+// sequences are scanned in their own order, 64 at a time.
 __device__ int find_sequence(const int32_t* qsl, const int32_t* prefix, int batch, int G,
                              int BM, int combos, int tile, int* local) {
   __shared__ int found_b, found_local;
@@ -349,28 +352,33 @@ __device__ int find_sequence(const int32_t* qsl, const int32_t* prefix, int batc
         n = ql > 0 ? (int)(((int64_t)ql * G + BM - 1) / BM) : 0;
         u = (int)min((int64_t)max(prefix[lane], 0) * G / BM, (int64_t)1 << 29);
       }
-      const bool by_tile =
-          (int64_t)wave_total(n) * combos <= (int64_t)tiles::kPagedTileOrderMax;
-      auto above = [&](int K) {
-        return by_tile ? min(max(u + n - K, 0), n) : (u > K ? n : 0);
-      };
-      // lo: more than `tile` tiles above it (or -1); hi: at most `tile`.
-      int lo = -1, hi = 1;
-      while (wave_total(above(hi)) > tile) {
-        lo = hi;
-        hi *= 2;
+      int last = wave_scan(n);
+      const int64_t wgs = (int64_t)__builtin_amdgcn_readlane(last, 63) * combos;
+      int here = n, before = 0, rank = tile;
+      const bool by_tile = wgs <= tiles::kPagedTileOrderMax;
+      const int u0 = __builtin_amdgcn_readfirstlane(u);
+      if (wgs > tiles::kPagedOneRound && (by_tile || __ballot(lane < batch && u != u0) != 0)) {
+        auto above = [&](int K) {
+          return by_tile ? min(max(u + n - K, 0), n) : (u + n > K ? n : 0);
+        };
+        // lo: more than `tile` tiles above it (or -1); hi: at most `tile`.
+        int lo = -1, hi = 1;
+        while (wave_total(above(hi)) > tile) {
+          lo = hi;
+          hi *= 2;
+        }
+        while (hi - lo > 1) {
+          const int mid = (lo + hi) >> 1;
+          if (wave_total(above(mid)) > tile)
+            lo = mid;
+          else
+            hi = mid;
+        }
+        before = above(hi);
+        rank = tile - wave_total(before);  // among the tiles at K = hi
+        here = above(hi - 1) - before;
+        last = wave_scan(here);
       }
-      while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (wave_total(above(mid)) > tile)
-          lo = mid;
-        else
-          hi = mid;
-      }
-      const int before = above(hi);
-      const int rank = tile - wave_total(before);  // among the tiles at K = hi
-      const int here = above(hi - 1) - before;
-      const int last = wave_scan(here);
       const uint64_t hit = __ballot(here > 0 && rank >= last - here && rank < last);
       if (hit) {
         fb = __ffsll((unsigned long long)hit) - 1;

@@ -128,6 +128,10 @@ __device__ __forceinline__ void attn_fwd_split_tile(const Prob& P, int row0, flo
   };
   auto issue_k = [&](int t, int bf) { issue_rows(t, kbuf(bf), BoolC<false>{}); };
   auto issue_v = [&](int t, int bf) { issue_rows(t, vbuf(bf), BoolC<true>{}); };
+  auto issue_kv = [&](int t, int bf) {
+    issue_k(t, bf);
+    issue_v(t, bf);
+  };
   // K operand of Sᵀ = K Qᵀ, chunk c: row lr, logical chunk 2c + lh.
   int koff[D / 16];
 #pragma unroll
@@ -221,14 +225,21 @@ __device__ __forceinline__ void attn_fwd_split_tile(const Prob& P, int row0, flo
   };
   // Waits for all but the n newest DMAs, and for the operand reads issued so
   // far before their buffer is overwritten.
+  // Builtins, not assembly: the compiler then knows the query loads have landed
+  // (it does not see the DMA) and puts no vmcnt(0) of its own into the loop,
+  // which would wait for the next tile (8% slower at [8, 125 x 1918, 12, 64]).
   auto wait_but = [](auto n) {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(n)::value) : "memory");
+    constexpr int N = decltype(n)::value;
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | (N >> 4) << 14);  // vmcnt(N)
+    asm volatile("" ::: "memory");
   };
-  auto wait_reads = []() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
+  auto wait_reads = []() {
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    asm volatile("" ::: "memory");
+  };
 
   if (t0 < t1) {
-    issue_k(t0, 0);
-    issue_v(t0, 0);
+    issue_kv(t0, 0);
   }
   // The lane's query row as B operand chunks (zero for rows past the last),
   // loaded while the first tile is in flight; one wait covers both, so the
@@ -247,8 +258,7 @@ __device__ __forceinline__ void attn_fwd_split_tile(const Prob& P, int row0, flo
     for (int t = t0; t < t1; ++t) {
       const int bf = (t - t0) & 1;
       if (t + 1 < t1) {
-        issue_k(t + 1, bf ^ 1);
-        issue_v(t + 1, bf ^ 1);
+        issue_kv(t + 1, bf ^ 1);
         wait_but(IntC<2 * S::BLKS>{});
       } else {
         wait_but(IntC<0>{});
@@ -258,8 +268,19 @@ __device__ __forceinline__ void attn_fwd_split_tile(const Prob& P, int row0, flo
       accumulate(bf);
       wait_reads();
     }
+  } else if constexpr (Prob::kRowStrided) {
+    // One buffer, dense rows (mostly from the L2): tile t + 1 is requested once
+    // tile t has been read.  (Requested in halves, as below, 1-2% slower.)
+    for (int t = t0; t < t1; ++t) {
+      if (t > t0) wait_but(IntC<0>{});
+      scores(0);
+      softmax(t);
+      accumulate(0);
+      wait_reads();
+      if (t + 1 < t1) issue_kv(t + 1, 0);
+    }
   } else {
-    // One buffer: K(t + 1) is requested once the scores of tile t have read
+    // One buffer, paged rows: K(t + 1) is requested once the scores of tile t have read
     // K(t), V(t + 1) once its products have read V(t), so each is in flight
     // for the other half of the tile's work.
     for (int t = t0; t < t1; ++t) {

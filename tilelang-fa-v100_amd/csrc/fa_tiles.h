@@ -203,16 +203,19 @@ constexpr int kSplitMaxRangeKeys = 8192;
 constexpr int kMaxSplits = 64;
 
 // ---- workgroup order of the paged kernels (fa_fwd.hip paged_order,
-// find_sequence): up to this many (tile, KV head, key range) workgroups, about
-// 8 rounds of the chip, every tile by its own reach; above it, whole sequences
-// by their history.  Evidence (us, same box, D = 128 unless noted, against
-// combo-major ranges of ids with sequences by history): 8 prompts of 512-4096
-// tokens, 16 / 2 heads 281 -> 255; 8 of 300-2048, 16 / 16 heads 110 -> 96; 8 of
-// 512-2048, 28 / 4 heads, D = 64 149 -> 129; the same after up to 4k keys, 16 / 2
-// heads, D = 256 988 -> 660; 2 chunks + 30 one-token sequences, 2 ranges 158 ->
-// 150.  Above the limit the tile order lost the K / V reuse in the L2: 8 prompts of
-// 512-4096 tokens, 32 / 8 heads (2400 workgroups) 467 -> 474, by history 460.
-constexpr int kPagedTileOrderMax = 2048;
+// find_sequence).  Up to kPagedOneRound (tile, KV head, key range) workgroups
+// start at once and go by sequence; up to kPagedTileOrderMax, two rounds, every
+// tile goes by its own reach; above, whole sequences by their reach where
+// histories differ, else in their own order.  Evidence (us, same box, D = 128
+// unless noted, against combo-major ranges of ids with sequences by history):
+// 8 prompts of 512-4096 tokens, 16 / 2 heads 281 -> 262; 8 of 300-2048, 16 / 16
+// heads 110 -> 105; 8 of 512-2048, 28 / 4 heads, D = 64 149 -> 143; the same after
+// up to 4k keys, 16 / 2 heads, D = 256 988 -> 680; 2 chunks + 30 one-token
+// sequences, 2 ranges 158 -> 150.  The tile order loses the K / V reuse in the
+// L2, so it stops at two rounds: 27 prompts of 356-712 tokens, 32 / 8 heads (1900
+// workgroups) 140 by sequence, 153 by tile; 8 of 512-4096 (2400) 467 and 474.
+constexpr int kPagedOneRound = 256;
+constexpr int kPagedTileOrderMax = 512;
 
 }  // namespace tiles
 }  // namespace fa
