@@ -149,6 +149,7 @@ size_t fa_bwd_workspace_bytes(const fa_bwd_args* args);
  * for callers that trade the dS tiles' memory for recomputing S and dP. */
 size_t fa_bwd_min_workspace_bytes(const fa_bwd_args* args);
 /* The workspace with which fa_bwd is fastest: fa_bwd_workspace_bytes plus,
+ * for window bands at head_dim 128 / 256, the dS tiles (dq from them), and
  * for problems with few (key tile, KV head) pairs, the fp32 partial dk / dv of
  * a dK / dV kernel split over the query rows (dk / dv then sum in another,
  * equally fixed, order).  Depends on the current device's CU count: query it
