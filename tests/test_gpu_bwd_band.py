@@ -21,6 +21,7 @@ from tilelang_fa_v100 import _dense, _lib
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 F16, BF16 = torch.float16, torch.bfloat16
+BIG = 2 ** 31 - 1
 
 CASES = [
     # (B, Sq, Sk, H, Hk, D, causal, window, dtype)
@@ -35,6 +36,12 @@ CASES = [
     (1, 2100, 2100, 2, 2, 128, True, (512, 0), BF16),     # several query blocks
     (1, 700, 700, 2, 2, 256, True, (129, 0), F16),
     (1, 300, 450, 2, 1, 256, False, (10, 90), F16),
+    # Bounds at the end of 32 bits, as "unbounded" is often written.
+    (1, 400, 400, 2, 2, 128, True, (BIG, 0), F16),
+    (1, 300, 500, 2, 1, 128, False, (-1, BIG), F16),
+    (1, 500, 300, 2, 2, 128, False, (BIG, BIG), F16),
+    (1, 500, 300, 2, 2, 128, True, (BIG - 100, 0), BF16),
+    (1, 290, 610, 2, 2, 256, False, (BIG, 3), F16),
 ]
 
 
@@ -70,6 +77,7 @@ def test_band_dq_paths_match_oracle_and_each_other(case):
     got, again = run(lib.fa_bwd_preferred_workspace_bytes), run(lib.fa_bwd_preferred_workspace_bytes)
     recomputed = run(lib.fa_bwd_min_workspace_bytes)
     want = ref.dense_attention_backward(q, k, v, do, causal=causal, window=window)
+    assert rel_l2(out, ref.dense_attention(q, k, v, causal=causal, window=window)[0]) < 1e-2, "out"
     for i, name in enumerate(("dq", "dk", "dv")):
         assert torch.equal(got[i], again[i]), f"{name}: two runs differ"
         if name != "dq":

@@ -99,11 +99,9 @@ template <int MODE>
 __host__ __device__ inline DsTiles<MODE> ds_tiles(int sq, int sk, int wl = -1, int wr = -1) {
   const int nq = (sq + 31) / 32, nk = (sk + 31) / 32;
   if constexpr (MODE == kMaskBand) {
-    // Bounds clamped to the lengths keep the sums in 32 bits; a bound at or past
-    // the other end hides nothing.
-    const int far = sq + sk, off = sk - sq;
-    const int c1 = wr < 0 ? nk + nq : floor_div32(31 + off + min(wr, far)) + 1;
-    const int cl = wl < 0 ? -nk - nq : floor_div32(off - min(wl, far));
+    const int off = sk - sq;  // (make_band keeps wl <= sk and wr <= sq)
+    const int c1 = wr < 0 ? nk + nq : floor_div32(31 + off + wr) + 1;
+    const int cl = wl < 0 ? -nk - nq : floor_div32(off - wl);
     return DsTiles<MODE>{nq, nk, c1, cl, max(min(nk, c1 - cl), 0)};
   } else {
     const int c1 = MODE == kMaskCausal ? floor_div32(31 + sk - sq) + 1 : nk;

@@ -322,9 +322,7 @@ void bwd_main_mfma_kernel(fa_bwd_args a, const float* stats, uint16_t* ds, float
   const int unm_hi = Sq - S::BQ;
   int b_act_lo = act_lo, b_act_hi = kNever, b_unm_lo = unm_lo, b_unm_hi = unm_hi;
   if constexpr (MODE == kMaskBand) {
-    // (Bounds at or past the lengths hide nothing; clamped, the sums stay in
-    // 32 bits.)
-    const int far = Sq + Sk, wr = min(band.wr, far), wl = min(band.wl, far);
+    const int wr = band.wr, wl = band.wl;
     if (kvw < Sk && wr >= 0) b_act_lo = kvw - (S::BQ - 1) - off - wr;
     if (wl >= 0) b_act_hi = kvw + 31 - off + wl;
     if (kvw + 32 <= Sk && wr >= 0) b_unm_lo = wkv_last - off - wr;

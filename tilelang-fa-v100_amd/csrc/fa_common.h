@@ -242,10 +242,13 @@ struct Band {
   }
 };
 
+// The bounds are clamped to the lengths: a left bound of seqlen_k or a right
+// bound of seqlen_q already hides nothing, and any larger one (up to 2^31 - 1)
+// would leave 32 bits in the sums with rows, keys and off.
 template <class Args>
 __device__ __host__ __forceinline__ Band make_band(const Args& a) {
-  const int wl = a.has_window ? a.window_left : -1;
-  const int wr = a.causal ? 0 : (a.has_window ? a.window_right : -1);
+  const int wl = a.has_window ? min(a.window_left, a.seqlen_k) : -1;
+  const int wr = a.causal ? 0 : (a.has_window ? min(a.window_right, a.seqlen_q) : -1);
   return Band{a.seqlen_k - a.seqlen_q, wl, wr};
 }
 
