@@ -61,3 +61,20 @@ def test_tile_orders_cover_every_tile(q_lens, heads):
     pf = torch.randint(0, 5, (len(q_lens),), generator=g).mul(50).tolist()
     c = make_case(33, q_lens, [p + q for p, q in zip(pf, q_lens)], pf, heads, heads, 64, page=16)
     run_split(c, 1)
+
+
+@pytest.mark.parametrize("q_lens,step,heads,dim", [
+    ([1] * 20 + [600] * 9, 300, 32, 64),          # 65 tiles x 32 heads: sequences by reach
+    ([1, 2, 129, 64, 0, 300] * 10, 300, 4, 64),   # 60 sequences, 320 workgroups: tiles by reach
+    ([200, 1, 370, 0, 129, 300] * 2, 0, 50, 64),  # no histories, 700 workgroups: tiles by reach
+    ([1100, 300, 0, 700], 0, 32, 128),            # no histories, 320 workgroups of one a CU
+    ([1100, 300, 0, 700], 0, 32, 256),            # 544 of one a CU: sequences in their own order
+    ([1030], 100, 40, 128),                       # one sequence: no search
+], ids=["by-sequence-reach", "by-reach", "two-rounds-d64", "two-rounds-d128", "own-order-d256",
+        "one"])
+def test_tile_orders_of_long_tiles(q_lens, step, heads, dim):
+    """The orders chosen from 1024 keys of reach on, and at two workgroups a CU."""
+    g = torch.Generator().manual_seed(41)
+    pf = torch.randint(0, 5, (len(q_lens),), generator=g).mul(step).tolist()
+    c = make_case(35, q_lens, [p + q for p, q in zip(pf, q_lens)], pf, heads, heads, dim, page=16)
+    run_split(c, 1)

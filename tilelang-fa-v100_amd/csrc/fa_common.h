@@ -297,6 +297,16 @@ __device__ __forceinline__ int wave_scan(int x) {
 __device__ __forceinline__ int wave_total(int x) {
   return __builtin_amdgcn_readlane(wave_scan(x), 63);
 }
+// Largest of the 64 lanes' values, which are not negative.
+__device__ __forceinline__ int wave_max_nonneg(int x) {
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true));
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true));
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true));
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true));
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, true));
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, true));
+  return __builtin_amdgcn_readlane(x, 63);
+}
 
 // Epilogue of the forward cores for one valid row: the lane holds
 // o[dt][4g + i] = O[row][32dt + 8g + 4lh + i] (unnormalised) and the row's

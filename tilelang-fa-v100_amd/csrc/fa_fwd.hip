@@ -300,7 +300,7 @@ struct PagedSplitRows : PagedRows {
 // first on every XCD and in every combo.  Ranges of ids that were contiguous
 // per XCD (combo-major) started each combo's long tiles when the one before
 // it ended, and with 1, 2 or 4 KV heads gave some XCDs only the long tiles and
-// others the short ones (figures at tiles::kPagedTileOrderMax).
+// others the short ones (figures at tiles::kPagedOrderMinKeys).
 struct SlotCombo {
   int slot, combo, combo_count;
 };
@@ -323,24 +323,30 @@ static int64_t paged_order_grid(int64_t slots, int64_t combos) {
   return (slots + f - 1) / f * f * combos;
 }
 
+// Compute units, and the workgroups they hold at once, for find_sequence.
+struct PagedOrder {
+  int cus, one_round;
+};
+
 // Finds the sequence owning slot `tile` in the varlen tile space where
 // sequence b has ceil(qlen_b * G / BM) tiles.  Returns b (or -1) and the
 // tile's index from the sequence's last (the one that sees most keys).
 // Up to 64 sequences, one per lane of wave 0, in one of three orders; u_b is the
 // history in units of a tile's rows, u_b + i + 1 the reach of tile i:
-//  * grids that start at once (tiles x combos up to kPagedOneRound), and larger
-//    ones than two rounds without histories to tell sequences apart: by sequence
-//    (the search below costs ~0.6 us a workgroup);
-//  * grids of two rounds (up to kPagedTileOrderMax): all tiles by decreasing
-//    reach, ties by sequence.  Sequence b has n_b(K) = clamp(u_b + ntiles_b - K,
-//    0, ntiles_b) tiles of reach above K;
-//  * larger grids: sequences by the reach of their last tile, longest first (the
-//    tiles of one share its K / V in the L2), n_b(K) = all or none.
-// For the last two a binary search for the smallest K with at most `tile` tiles
-// above it, and the slot's rank among those at K, name the tile.  More
-// sequences are scanned in their own order, 64 at a time.
+//  * by sequence, where the order costs nothing (no more tiles x combos than
+//    CUs, or than start at once with histories alike; a single sequence), has
+//    nothing to go by (more than two rounds, histories alike) or would not pay
+//    for its search (kPagedOrderMinKeys);
+//  * up to two rounds: all tiles by decreasing reach, ties by sequence.
+//    Sequence b has n_b(K) = clamp(u_b + ntiles_b - K, 0, ntiles_b) tiles of
+//    reach above K;
+//  * more than two rounds: sequences by the reach of their last tile, longest
+//    first (the tiles of one share its K / V in the L2), n_b(K) = all or none.
+// For the last two a search for the smallest K with at most `tile` tiles above
+// it, and the slot's rank among those at K, name the tile.  More sequences are
+// scanned in their own order, 64 at a time.
 __device__ int find_sequence(const int32_t* qsl, const int32_t* prefix, int batch, int G,
-                             int BM, int combos, int tile, int* local) {
+                             int BM, int combos, PagedOrder order, int tile, int* local) {
   __shared__ int found_b, found_local;
   if (wave_id() == 0) {
     const int lane = threadIdx.x & 63;
@@ -353,31 +359,36 @@ __device__ int find_sequence(const int32_t* qsl, const int32_t* prefix, int batc
         u = (int)min((int64_t)max(prefix[lane], 0) * G / BM, (int64_t)1 << 29);
       }
       int last = wave_scan(n);
-      const int64_t wgs = (int64_t)__builtin_amdgcn_readlane(last, 63) * combos;
+      const int total = __builtin_amdgcn_readlane(last, 63);
+      const int64_t wgs = (int64_t)total * combos;
       int here = n, before = 0, rank = tile;
-      const bool by_tile = wgs <= tiles::kPagedTileOrderMax;
-      const int u0 = __builtin_amdgcn_readfirstlane(u);
-      if (wgs > tiles::kPagedOneRound && (by_tile || __ballot(lane < batch && u != u0) != 0)) {
-        auto above = [&](int K) {
-          return by_tile ? min(max(u + n - K, 0), n) : (u + n > K ? n : 0);
-        };
-        // lo: more than `tile` tiles above it (or -1); hi: at most `tile`.
-        int lo = -1, hi = 1;
-        while (wave_total(above(hi)) > tile) {
-          lo = hi;
-          hi *= 2;
+      const bool by_tile = wgs <= 2 * (int64_t)order.one_round;
+      const uint64_t some = __ballot(n > 0);
+      if (wgs > order.cus && tile < total && (some & (some - 1)) != 0) {
+        const int u0 = __builtin_amdgcn_readlane(u, __ffsll((unsigned long long)some) - 1);
+        const bool differ = __ballot(n > 0 && u != u0) != 0;
+        int hi = wave_max_nonneg(u + n);
+        const bool far = (int64_t)hi * BM >= (int64_t)tiles::kPagedOrderMinKeys * G;
+        if (differ ? far : by_tile && wgs > order.one_round && (far || order.one_round > order.cus)) {
+          auto above = [&](int K) {
+            return by_tile ? min(max(u + n - K, 0), n) : (u + n > K ? n : 0);
+          };
+          // lo: all tiles lie above the least history; hi: none above the
+          // longest reach.
+          constexpr int kFar = 1 << 29;  // u's bound
+          int lo = kFar - wave_max_nonneg(n > 0 ? kFar - u : 0);
+          while (hi - lo > 1) {
+            const int mid = (int)(((unsigned)lo + (unsigned)hi) >> 1);
+            if (wave_total(above(mid)) > tile)
+              lo = mid;
+            else
+              hi = mid;
+          }
+          before = above(hi);
+          rank = tile - wave_total(before);  // among the tiles at K = hi
+          here = above(hi - 1) - before;
+          last = wave_scan(here);
         }
-        while (hi - lo > 1) {
-          const int mid = (lo + hi) >> 1;
-          if (wave_total(above(mid)) > tile)
-            lo = mid;
-          else
-            hi = mid;
-        }
-        before = above(hi);
-        rank = tile - wave_total(before);  // among the tiles at K = hi
-        here = above(hi - 1) - before;
-        last = wave_scan(here);
       }
       const uint64_t hit = __ballot(here > 0 && rank >= last - here && rank < last);
       if (hit) {
@@ -504,7 +515,7 @@ __device__ __forceinline__ void run_paged_tile(const fa_paged_args& a, int rows,
 
 template <class T, int D, bool PP>
 __global__ __launch_bounds__((FwdKernelCfg<D, PP>::THREADS), (FwdKernelCfg<D, PP>::WAVES_PER_EU))
-void fwd_paged_kernel(fa_paged_args a) {
+void fwd_paged_kernel(fa_paged_args a, PagedOrder order) {
   using S = FwdKernelCfg<D, PP>;
   const int G = a.num_heads / a.num_kv_heads;
   const SlotCombo sc = paged_order(blockIdx.x, a.num_kv_heads);
@@ -512,7 +523,7 @@ void fwd_paged_kernel(fa_paged_args a) {
 
   int local = 0;
   const int b = find_sequence(a.query_start_loc, a.prefix_kv_lens, a.batch, G, S::BM,
-                              sc.combo_count, slot, &local);
+                              sc.combo_count, order, slot, &local);
   if (b < 0) return;
   const int qs = a.query_start_loc[b];
   const int qlen = a.query_start_loc[b + 1] - qs;
@@ -530,7 +541,8 @@ void fwd_paged_kernel(fa_paged_args a) {
 // 128.
 template <class T, int D, bool PP>
 __global__ __launch_bounds__((FwdKernelCfg<D, PP>::THREADS), (FwdKernelCfg<D, PP>::WAVES_PER_EU))
-void fwd_paged_split_kernel(fa_paged_args a, int nsplit, float* po, float* plse) {
+void fwd_paged_split_kernel(fa_paged_args a, PagedOrder order, int nsplit, float* po,
+                            float* plse) {
   using S = FwdKernelCfg<D, PP>;
   const int G = a.num_heads / a.num_kv_heads;
   const SlotCombo sc = paged_order(blockIdx.x, a.num_kv_heads * nsplit);
@@ -539,7 +551,7 @@ void fwd_paged_split_kernel(fa_paged_args a, int nsplit, float* po, float* plse)
 
   int local = 0;
   const int b = find_sequence(a.query_start_loc, a.prefix_kv_lens, a.batch, G, S::BM,
-                              sc.combo_count, slot, &local);
+                              sc.combo_count, order, slot, &local);
   if (b < 0) return;
   const int qs = a.query_start_loc[b];
   const int qlen = a.query_start_loc[b + 1] - qs;
@@ -705,16 +717,18 @@ static hipError_t launch_paged_pp(const fa_paged_args& a, int nsplit, void* ws,
                                   hipStream_t st) {
   const unsigned grid = (unsigned)paged_order_grid(
       paged_grid_slots(a), (int64_t)a.num_kv_heads * std::max(nsplit, 1));
+  const int cus = device_cu_count();
+  const PagedOrder order{cus, cus * FwdKernelCfg<D, PP>::WG_PER_CU};
   if (nsplit <= 1) {
     hipLaunchKernelGGL((fwd_paged_kernel<T, D, PP>), dim3(grid),
-                       dim3(FwdKernelCfg<D, PP>::THREADS), 0, st, a);
+                       dim3(FwdKernelCfg<D, PP>::THREADS), 0, st, a, order);
     return hipGetLastError();
   }
   const size_t rows = (size_t)nsplit * a.num_heads * a.num_tokens;
   float* po = static_cast<float*>(ws);
   float* plse = po + rows * D;
   hipLaunchKernelGGL((fwd_paged_split_kernel<T, D, PP>), dim3(grid),
-                     dim3(FwdKernelCfg<D, PP>::THREADS), 0, st, a, nsplit, po, plse);
+                     dim3(FwdKernelCfg<D, PP>::THREADS), 0, st, a, order, nsplit, po, plse);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const int64_t items = (int64_t)a.num_heads * a.num_tokens;

@@ -203,19 +203,25 @@ constexpr int kSplitMaxRangeKeys = 8192;
 constexpr int kMaxSplits = 64;
 
 // ---- workgroup order of the paged kernels (fa_fwd.hip paged_order,
-// find_sequence).  Up to kPagedOneRound (tile, KV head, key range) workgroups
-// start at once and go by sequence; up to kPagedTileOrderMax, two rounds, every
-// tile goes by its own reach; above, whole sequences by their reach where
-// histories differ, else in their own order.  Evidence (us, same box, D = 128
-// unless noted, against combo-major ranges of ids with sequences by history):
-// 8 prompts of 512-4096 tokens, 16 / 2 heads 281 -> 262; 8 of 300-2048, 16 / 16
-// heads 110 -> 105; 8 of 512-2048, 28 / 4 heads, D = 64 149 -> 143; the same after
-// up to 4k keys, 16 / 2 heads, D = 256 988 -> 680; 2 chunks + 30 one-token
-// sequences, 2 ranges 158 -> 150.  The tile order loses the K / V reuse in the
-// L2, so it stops at two rounds: 27 prompts of 356-712 tokens, 32 / 8 heads (1900
-// workgroups) 140 by sequence, 153 by tile; 8 of 512-4096 (2400) 467 and 474.
-constexpr int kPagedOneRound = 256;
-constexpr int kPagedTileOrderMax = 512;
+// find_sequence).  Up to two rounds of (tile, KV head, key range) workgroups
+// (CUs x workgroups per CU is one) every tile goes by its own reach; above, whole
+// sequences by their reach where histories differ, else in their own order.
+// Evidence (us, same box, D = 128 unless noted, against combo-major ranges of ids
+// with sequences by history): 8 prompts of 512-4096 tokens, 16 / 2 heads 281 -> 262;
+// 8 of 300-2048, 16 / 16 heads 110 -> 105; 8 of 512-2048, 28 / 4 heads, D = 64
+// 149 -> 143; the same after up to 4k keys, 16 / 2 heads, D = 256 988 -> 680; 2
+// chunks + 30 one-token sequences, 2 ranges 158 -> 150.  The tile order loses the
+// K / V reuse in the L2, so it stops at two rounds: 27 prompts of 356-712 tokens,
+// 32 / 8 heads (1900 workgroups) 140 by sequence, 153 by tile; 8 of 512-4096 (2400)
+// 467 and 474.
+// The search for a workgroup's tile takes ~0.08 us a halving, 0.5-1 us in all,
+// which a CU's only workgroup waits for: reaches below kPagedOrderMinKeys keys go
+// by sequence (searched / by sequence: 2 prompts of 434-868 tokens, 64 / 8 heads
+// 37.4 / 35.8, 2 of 535-1070, 32 / 8, D = 256 47.1 / 44.7; 23 chunks of 23-46
+// tokens after 0.8-3.1k keys, 32 / 8, D = 64 61 / 68).  Two workgroups a CU (D = 64)
+// hide it, and their second round pays for it at any reach: 14 prompts of 185-370,
+// 28 / 4 heads 27.1 / 29.0, 4 of 736-1472, 16 / 16 heads 33.9 / 40.4.
+constexpr int kPagedOrderMinKeys = 1024;
 
 }  // namespace tiles
 }  // namespace fa
