@@ -67,13 +67,14 @@ def test_tile_orders_cover_every_tile(q_lens, heads):
     ([1] * 20 + [600] * 9, 300, 32, 64),          # 65 tiles x 32 heads: sequences by reach
     ([1, 2, 129, 64, 0, 300] * 10, 300, 4, 64),   # 60 sequences, 320 workgroups: tiles by reach
     ([200, 1, 370, 0, 129, 300] * 2, 0, 50, 64),  # no histories, 700 workgroups: tiles by reach
-    ([1100, 300, 0, 700], 0, 32, 128),            # no histories, 320 workgroups of one a CU
-    ([1100, 300, 0, 700], 0, 32, 256),            # 544 of one a CU: sequences in their own order
-    ([1030], 100, 40, 128),                       # one sequence: no search
+    ([1100, 300, 0, 700], 0, 32, 128),            # no histories, 320 workgroups: tiles by reach
+    ([1100, 300, 0, 700], 0, 32, 256),            # 544, one a CU: sequences in their own order
+    ([500, 0, 530], 0, 66, 128),                  # two short prompts: no search
+    ([500, 0, 530], 100, 66, 128),                # two histories
 ], ids=["by-sequence-reach", "by-reach", "two-rounds-d64", "two-rounds-d128", "own-order-d256",
-        "one"])
-def test_tile_orders_of_long_tiles(q_lens, step, heads, dim):
-    """The orders chosen from 1024 keys of reach on, and at two workgroups a CU."""
+        "two", "two-histories"])
+def test_tile_orders_by_rounds(q_lens, step, heads, dim):
+    """Each order, at one workgroup a CU (D = 128, 256) and two (D = 64)."""
     g = torch.Generator().manual_seed(41)
     pf = torch.randint(0, 5, (len(q_lens),), generator=g).mul(step).tolist()
     c = make_case(35, q_lens, [p + q for p, q in zip(pf, q_lens)], pf, heads, heads, dim, page=16)

@@ -300,7 +300,7 @@ struct PagedSplitRows : PagedRows {
 // first on every XCD and in every combo.  Ranges of ids that were contiguous
 // per XCD (combo-major) started each combo's long tiles when the one before
 // it ended, and with 1, 2 or 4 KV heads gave some XCDs only the long tiles and
-// others the short ones (figures at tiles::kPagedOrderMinKeys).
+// others the short ones (figures in fa_tiles.h).
 struct SlotCombo {
   int slot, combo, combo_count;
 };
@@ -323,7 +323,8 @@ static int64_t paged_order_grid(int64_t slots, int64_t combos) {
   return (slots + f - 1) / f * f * combos;
 }
 
-// Compute units, and the workgroups they hold at once, for find_sequence.
+// Compute units, and the workgroups they hold at once, for find_sequence (figures
+// in fa_tiles.h).
 struct PagedOrder {
   int cus, one_round;
 };
@@ -333,10 +334,10 @@ struct PagedOrder {
 // tile's index from the sequence's last (the one that sees most keys).
 // Up to 64 sequences, one per lane of wave 0, in one of three orders; u_b is the
 // history in units of a tile's rows, u_b + i + 1 the reach of tile i:
-//  * by sequence, where the order costs nothing (no more tiles x combos than
-//    CUs, or than start at once with histories alike; a single sequence), has
-//    nothing to go by (more than two rounds, histories alike) or would not pay
-//    for its search (kPagedOrderMinKeys);
+//  * by sequence, each from its longest tile: grids of no more workgroups (tiles x
+//    combos) than CUs, a single sequence or two short prompts (the search below
+//    costs 0.5-1 us a workgroup), and more than two rounds without histories to
+//    tell sequences apart;
 //  * up to two rounds: all tiles by decreasing reach, ties by sequence.
 //    Sequence b has n_b(K) = clamp(u_b + ntiles_b - K, 0, ntiles_b) tiles of
 //    reach above K;
@@ -364,19 +365,19 @@ __device__ int find_sequence(const int32_t* qsl, const int32_t* prefix, int batc
       int here = n, before = 0, rank = tile;
       const bool by_tile = wgs <= 2 * (int64_t)order.one_round;
       const uint64_t some = __ballot(n > 0);
-      if (wgs > order.cus && tile < total && (some & (some - 1)) != 0) {
+      if (wgs > order.cus && tile < total && __popcll(some) > 1) {
         const int u0 = __builtin_amdgcn_readlane(u, __ffsll((unsigned long long)some) - 1);
-        const bool differ = __ballot(n > 0 && u != u0) != 0;
-        int hi = wave_max_nonneg(u + n);
-        const bool far = (int64_t)hi * BM >= (int64_t)tiles::kPagedOrderMinKeys * G;
-        if (differ ? far : by_tile && wgs > order.one_round && (far || order.one_round > order.cus)) {
+        auto reach = [&]() { return wave_max_nonneg(u + n); };
+        if (__ballot(n > 0 && u != u0) != 0 ||
+            (by_tile && (__popcll(some) > 2 ||
+                         (int64_t)reach() * BM >= (int64_t)tiles::kPagedOrderPairKeys * G))) {
           auto above = [&](int K) {
             return by_tile ? min(max(u + n - K, 0), n) : (u + n > K ? n : 0);
           };
           // lo: all tiles lie above the least history; hi: none above the
           // longest reach.
           constexpr int kFar = 1 << 29;  // u's bound
-          int lo = kFar - wave_max_nonneg(n > 0 ? kFar - u : 0);
+          int lo = kFar - wave_max_nonneg(n > 0 ? kFar - u : 0), hi = reach();
           while (hi - lo > 1) {
             const int mid = (int)(((unsigned)lo + (unsigned)hi) >> 1);
             if (wave_total(above(mid)) > tile)

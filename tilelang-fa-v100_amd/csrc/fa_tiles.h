@@ -214,14 +214,15 @@ constexpr int kMaxSplits = 64;
 // K / V reuse in the L2, so it stops at two rounds: 27 prompts of 356-712 tokens,
 // 32 / 8 heads (1900 workgroups) 140 by sequence, 153 by tile; 8 of 512-4096 (2400)
 // 467 and 474.
-// The search for a workgroup's tile takes ~0.08 us a halving, 0.5-1 us in all,
-// which a CU's only workgroup waits for: reaches below kPagedOrderMinKeys keys go
-// by sequence (searched / by sequence: 2 prompts of 434-868 tokens, 64 / 8 heads
-// 37.4 / 35.8, 2 of 535-1070, 32 / 8, D = 256 47.1 / 44.7; 23 chunks of 23-46
-// tokens after 0.8-3.1k keys, 32 / 8, D = 64 61 / 68).  Two workgroups a CU (D = 64)
-// hide it, and their second round pays for it at any reach: 14 prompts of 185-370,
-// 28 / 4 heads 27.1 / 29.0, 4 of 736-1472, 16 / 16 heads 33.9 / 40.4.
-constexpr int kPagedOrderMinKeys = 1024;
+// The search for a workgroup's tile takes 0.5-1 us, so a single sequence and two
+// prompts below kPagedOrderPairKeys go without it (searched / by sequence: one of
+// 535-1070 tokens, 64 / 8 heads, D = 256 47.3 / 45.4; two of 434-868, 64 / 8 37.4 /
+// 35.8), while two longer ones or three and more gain by it (two of 941-1882, 16 / 16,
+// D = 64 41.5 / 47.2; 11 of 411-822, 16 / 2 41.2 / 48.0; 5 of 169-338, 64 / 8, D = 64
+// 21.5 / 24.5), as do two histories (two of 100-200 after 8-31k keys, 28 / 4, 6 ranges
+// 117 / 144).  Two rounds are 1024 workgroups at D = 64, which runs two a CU (14 of
+// 185-370, 28 / 4 27.1 by tile, 29.0 by sequence; 4 of 736-1472, 16 / 16 33.9, 40.4).
+constexpr int kPagedOrderPairKeys = 1024;
 
 }  // namespace tiles
 }  // namespace fa
