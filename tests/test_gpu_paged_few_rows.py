@@ -28,6 +28,14 @@ CASES = [
     ([1, 32, 1], [33, 77, 2000], 8, 8, 64, 64, F16, True, 50, -1, 2),
     ([1, 4, 5, 1], [1, 127, 131, 1500], 16, 2, 256, 16, F16, True, -1, -1, 1),
     ([1, 3, 140], [2000, 31, 170], 16, 2, 256, 32, BF16, True, -1, -1, 3),
+    # Around the least count that is split, 384 keys (of a range), and the
+    # edges of tiles and of the waves' ranges above it.
+    ([1, 8, 9, 1, 1, 1], [383, 384, 385, 415, 513, 767], 16, 4, 128, 16, F16, True, -1, -1, 1),
+    ([1, 1, 8, 2, 1], [1151, 1152, 1154, 1249, 1700], 16, 4, 128, 32, BF16, True, -1, -1, 3),
+    ([1, 1, 8, 1], [383, 384, 417, 2051], 8, 2, 64, 16, F16, True, -1, -1, 1),
+    ([1, 3, 1], [384, 497, 777], 16, 2, 256, 16, F16, True, -1, -1, 1),
+    ([1] * 20, [384 + 5 * i for i in range(20)], 16, 16, 256, 16, F16, True, -1, -1, 1),  # > CUs
+    ([1, 1, 900], [900, 2000, 1000], 64, 8, 128, 16, F16, True, -1, -1, 1),  # mostly full tiles
 ]
 
 

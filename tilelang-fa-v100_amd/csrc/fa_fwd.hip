@@ -470,27 +470,27 @@ __device__ __forceinline__ void paged_rows(const Args& a, int hk, int b, int qs,
   P.wk = a.window_k;
 }
 
-// One row tile of a paged problem; setup(args, P) fills the problem from the
-// kernel's arguments.  A tile of at most 32 rows (a decoding sequence in a
-// prefill batch, or the last rows of a prompt) would keep one wave of the
-// row-tile cores busy, serially over the keys; its keys are split over the
-// waves instead (fa_fwd_split.h; pages of at least 16 keys, strides that fit
-// its 32-bit lane offsets).  Each branch sets up its own problem, the few-row
-// one from arguments the compiler reloads: with one problem for both, its
-// scalars stayed live across the ping-pong core and spilled in its loop (49
-// spilled SGPRs against 13, C5-size chunked prefill 0.7% slower).
-template <class T, int D, bool PP, class Prob, class Setup>
-__device__ __forceinline__ void run_paged_tile(const fa_paged_args& a, int rows, int row0,
-                                               Setup setup) {
+// One row tile of a paged problem, which sees up to keys() keys; setup(args, P)
+// fills the problem from the kernel's arguments.  A tile of at most 32 rows (a
+// decoding sequence in a prefill batch, or the last rows of a prompt) would
+// keep one wave of the row-tile cores busy, serially over the keys; with FEW
+// its keys, from kPagedFewMinKeys on, are split over the waves instead
+// (fa_fwd_split.h).  Each branch sets up its own problem, the few-row one from
+// arguments the compiler reloads: with one problem for both, its scalars stayed
+// live across the ping-pong core and spilled in its loop (49 spilled SGPRs
+// against 13, C5-size chunked prefill 0.7% slower).  The launcher leaves FEW out
+// where tiles are mostly full (paged_few_rows): the branch costs the row-tile
+// cores registers (head_dim 256 242 -> 256 VGPRs).
+template <class T, int D, bool PP, bool FEW, class Prob, class Keys, class Setup>
+__device__ __forceinline__ void run_paged_tile(const fa_paged_args& a, int rows, Keys keys,
+                                               int row0, Setup setup) {
   using C = FwdKernelCfg<D, PP>;
-  if constexpr (D == 64 || (PP && (D == 128 || D == 256))) {
+  if constexpr (FEW) {
     constexpr int NW = C::THREADS / 64;
     constexpr int kSplitLds = FwdSplitShape<D, NW>::LDS;
     constexpr int kLds = kSplitLds > C::LDS_BYTES ? kSplitLds : C::LDS_BYTES;
     __shared__ __attribute__((aligned(16))) char smem[kLds];
-    constexpr int64_t kMaxSlot = 1 << 24;
-    if (rows <= 32 && (PP || (a.page_size >= 16 && a.k_stride[1] < kMaxSlot &&
-                              a.v_stride[1] < kMaxSlot))) {
+    if (rows <= 32 && keys() >= tiles::kPagedFewMinKeys) {
       const auto* ap = kernel_args<fa_paged_args>();
       Prob P;
       setup(*ap, P);
@@ -514,7 +514,7 @@ __device__ __forceinline__ void run_paged_tile(const fa_paged_args& a, int rows,
   }
 }
 
-template <class T, int D, bool PP>
+template <class T, int D, bool PP, bool FEW>
 __global__ __launch_bounds__((FwdKernelCfg<D, PP>::THREADS), (FwdKernelCfg<D, PP>::WAVES_PER_EU))
 void fwd_paged_kernel(fa_paged_args a, PagedOrder order) {
   using S = FwdKernelCfg<D, PP>;
@@ -532,15 +532,15 @@ void fwd_paged_kernel(fa_paged_args a, PagedOrder order) {
   // Later tiles of a causal sequence see more keys: run them first.
   const int tile = ntiles - 1 - local;
   const int row0 = tile * S::BM;
-  run_paged_tile<T, D, PP, PagedRows>(
-      a, qlen * G - row0, row0,
+  run_paged_tile<T, D, PP, FEW, PagedRows>(
+      a, qlen * G - row0, [&a, b] { return a.seq_lens[b]; }, row0,
       [=](const auto& args, PagedRows& P) { paged_rows(args, hk, b, qs, qlen, P); });
 }
 
 // Split-KV variant: workgroup (KV head, split, tile slot); the splits of a
 // sequence cover its keys in ranges of ceil(seq_len / nsplit) rounded up to
 // 128.
-template <class T, int D, bool PP>
+template <class T, int D, bool PP, bool FEW>
 __global__ __launch_bounds__((FwdKernelCfg<D, PP>::THREADS), (FwdKernelCfg<D, PP>::WAVES_PER_EU))
 void fwd_paged_split_kernel(fa_paged_args a, PagedOrder order, int nsplit, float* po,
                             float* plse) {
@@ -559,8 +559,9 @@ void fwd_paged_split_kernel(fa_paged_args a, PagedOrder order, int nsplit, float
   const int ntiles = (int)(((int64_t)qlen * G + S::BM - 1) / S::BM);
   const int tile = ntiles - 1 - local;
   const int row0 = tile * S::BM;
-  run_paged_tile<T, D, PP, PagedSplitRows>(
-      a, qlen * G - row0, row0, [=](const auto& args, PagedSplitRows& P) {
+  run_paged_tile<T, D, PP, FEW, PagedSplitRows>(
+      a, qlen * G - row0, [&a, b, nsplit] { return a.seq_lens[b] / nsplit; }, row0,
+      [=](const auto& args, PagedSplitRows& P) {
         paged_rows(args, hk, b, qs, qlen, P);
         const int chunk = ((P.seq_len + nsplit - 1) / nsplit + 127) / 128 * 128;
         P.split_lo = split * chunk;
@@ -713,7 +714,37 @@ int paged_grid_slots(const fa_paged_args& a) {
   return (int)((rows + bm - 1) / bm + a.batch);
 }
 
-template <class T, int D, bool PP>
+// Workgroups of a paged problem before any split: the row tiles of all tokens
+// together, but at least one per sequence (every sequence with tokens has a
+// tile of its own), times the KV heads.
+struct PagedTiles {
+  int64_t rows, seqs, wgs;
+};
+static PagedTiles paged_tiles(const fa_paged_args& a) {
+  const int64_t rows = (int64_t)a.num_tokens * (a.num_heads / a.num_kv_heads);
+  const int64_t seqs = std::max(1, std::min(a.batch, a.num_tokens));
+  const int bm = paged_block_rows(a);
+  return {rows, seqs, std::max<int64_t>(seqs, (rows + bm - 1) / bm) * a.num_kv_heads};
+}
+
+// Whether few-row tiles get the key-split core, from sizes alone: pages and
+// strides it can address (those of the ping-pong cores), and a batch in which
+// such tiles can matter: at most kPagedFewMaxTiles full tiles per sequence,
+// and more than the last rows of a single prompt.  Its workgroups at head_dim
+// 256 have half the bytes in flight of the row-tile core's (one buffer in LDS),
+// so once every CU has one, and with them the memory is busy, they lose
+// (figures at kPagedFewMinKeys), except in batches that are mostly full tiles.
+static bool paged_few_rows(const fa_paged_args& a, int nsplit) {
+  const int64_t lim = int64_t(1) << 24;
+  if (a.head_dim > 256 || a.page_size < 16 || a.k_stride[1] >= lim || a.v_stride[1] >= lim)
+    return false;
+  const PagedTiles t = paged_tiles(a);
+  const int64_t bm = paged_block_rows(a);
+  if (t.rows > tiles::kPagedFewMaxTiles * bm * t.seqs || (t.seqs == 1 && t.rows > 32)) return false;
+  return a.head_dim != 256 || t.wgs * nsplit < device_cu_count() || t.rows > bm * t.seqs;
+}
+
+template <class T, int D, bool PP, bool FEW>
 static hipError_t launch_paged_pp(const fa_paged_args& a, int nsplit, void* ws,
                                   hipStream_t st) {
   const unsigned grid = (unsigned)paged_order_grid(
@@ -721,14 +752,14 @@ static hipError_t launch_paged_pp(const fa_paged_args& a, int nsplit, void* ws,
   const int cus = device_cu_count();
   const PagedOrder order{cus, cus * FwdKernelCfg<D, PP>::WG_PER_CU};
   if (nsplit <= 1) {
-    hipLaunchKernelGGL((fwd_paged_kernel<T, D, PP>), dim3(grid),
+    hipLaunchKernelGGL((fwd_paged_kernel<T, D, PP, FEW>), dim3(grid),
                        dim3(FwdKernelCfg<D, PP>::THREADS), 0, st, a, order);
     return hipGetLastError();
   }
   const size_t rows = (size_t)nsplit * a.num_heads * a.num_tokens;
   float* po = static_cast<float*>(ws);
   float* plse = po + rows * D;
-  hipLaunchKernelGGL((fwd_paged_split_kernel<T, D, PP>), dim3(grid),
+  hipLaunchKernelGGL((fwd_paged_split_kernel<T, D, PP, FEW>), dim3(grid),
                      dim3(FwdKernelCfg<D, PP>::THREADS), 0, st, a, order, nsplit, po, plse);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
@@ -741,9 +772,13 @@ static hipError_t launch_paged_pp(const fa_paged_args& a, int nsplit, void* ws,
 template <class T, int D>
 static hipError_t launch_paged(const fa_paged_args& a, int nsplit, void* ws, hipStream_t st) {
   if constexpr (D == 128 || D == 256) {
-    if (paged_pingpong(a)) return launch_paged_pp<T, D, true>(a, nsplit, ws, st);
+    if (paged_pingpong(a))
+      return paged_few_rows(a, nsplit) ? launch_paged_pp<T, D, true, true>(a, nsplit, ws, st)
+                                       : launch_paged_pp<T, D, true, false>(a, nsplit, ws, st);
   }
-  return launch_paged_pp<T, D, false>(a, nsplit, ws, st);
+  if constexpr (D == 64)
+    if (paged_few_rows(a, nsplit)) return launch_paged_pp<T, D, false, true>(a, nsplit, ws, st);
+  return launch_paged_pp<T, D, false, false>(a, nsplit, ws, st);
 }
 
 template <class T>
@@ -774,16 +809,9 @@ size_t paged_split_workspace_bytes(const fa_paged_args& a, int nsplit) {
   return rows * a.head_dim * sizeof(float) + rows * sizeof(float) + 256;
 }
 
-// Split count from sizes alone (no device data).  Workgroups unsplit: the row
-// tiles of all tokens together, but at least one per sequence (every sequence
-// with tokens has a tile of its own), times the KV heads.
+// Split count from sizes alone (no device data).
 int paged_num_splits(const fa_paged_args& a) {
-  const int G = a.num_heads / a.num_kv_heads;
-  const int64_t rows = (int64_t)a.num_tokens * G;
-  const int64_t seqs = std::max(1, std::min(a.batch, a.num_tokens));
-  const int64_t tiles = std::max<int64_t>(
-      seqs, (rows + paged_block_rows(a) - 1) / paged_block_rows(a));
-  const int64_t wgs = tiles * a.num_kv_heads;
+  const auto [rows, seqs, wgs] = paged_tiles(a);
   const int64_t kv_cap = (int64_t)a.max_blocks * a.page_size;
   const int cus = device_cu_count();
   if (kv_cap < tiles::kSplitMinKeys || 2 * wgs >= 3 * cus) return 1;

@@ -224,5 +224,20 @@ constexpr int kMaxSplits = 64;
 // 185-370, 28 / 4 27.1 by tile, 29.0 by sequence; 4 of 736-1472, 16 / 16 33.9, 40.4).
 constexpr int kPagedOrderPairKeys = 1024;
 
+// ---- paged tiles of at most 32 rows (fa_fwd.hip run_paged_tile, paged_few_rows):
+// their keys are split over the workgroup's waves from kPagedFewMinKeys keys (of
+// the tile's range) on, in batches of at most kPagedFewMaxTiles full tiles per
+// sequence.  Evidence (us, one-token sequences, row-tile / key-split core, one
+// range): D = 128, 32 / 8 heads, 16 sequences of 512 / 2048 / 8192 keys 19.7 / 18.1,
+// 48.7 / 31.1, 190 / 125; 128 of 128 / 256 / 512 / 2048 keys 33.2 / 38.5, 45.1 / 47.0,
+// 67.5 / 58.5, 228 / 196.  D = 64, 16 of 1024 / 8192 23.8 / 17.3, 122 / 65; 128 of 256 /
+// 512 24.3 / 24.3, 34.0 / 31.8.  D = 256 (fewer workgroups than CUs only): 16 of 1024 /
+// 8192 45.5 / 32.3, 288 / 210; 32 (256 workgroups) 48.7 / 49.5, 347 / 381; 64 101 / 105,
+// 682 / 747.  Mixed with chunks, D = 128: 3 sequences, one of a token, 32 / 8 heads, 644
+// rows a sequence, 7k keys 75 / 65; D = 256: 39 of 3-9k keys, 20 of them chunks of 116
+// tokens 767 / 687.
+constexpr int kPagedFewMinKeys = 384;
+constexpr int kPagedFewMaxTiles = 8;
+
 }  // namespace tiles
 }  // namespace fa
