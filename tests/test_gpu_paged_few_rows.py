@@ -87,3 +87,11 @@ def test_tile_orders_by_rounds(q_lens, step, heads, dim):
     pf = torch.randint(0, 5, (len(q_lens),), generator=g).mul(step).tolist()
     c = make_case(35, q_lens, [p + q for p, q in zip(pf, q_lens)], pf, heads, heads, dim, page=16)
     run_split(c, 1)
+
+
+@pytest.mark.parametrize("Hkv,splits,dim", [(1, 2, 128), (2, 3, 128), (3, 5, 64), (8, 2, 128),
+                                            (5, 2, 256)])
+def test_ranges_in_turn_cover_every_tile(Hkv, splits, dim):
+    """Split prompts of at least 512 new tokens a sequence: one key range after the other."""
+    c = make_case(43, [1300, 0, 600], [1700, 5, 640], [400, 5, 40], Hkv, Hkv, dim, page=16)
+    run_split(c, splits)

@@ -302,19 +302,19 @@ struct PagedSplitRows : PagedRows {
 // it ended, and with 1, 2 or 4 KV heads gave some XCDs only the long tiles and
 // others the short ones (figures in fa_tiles.h).
 struct SlotCombo {
-  int slot, combo, combo_count;
+  int slot, combo;
 };
 constexpr int kOrderXcds = 8;
 __device__ __forceinline__ SlotCombo paged_order(int wg, int combos) {
   const int x = wg % kOrderXcds, l = wg / kOrderXcds;
   if (combos % kOrderXcds == 0) {
     const int per = combos / kOrderXcds;
-    return {l / per, x * per + l % per, combos};
+    return {l / per, x * per + l % per};
   }
   if (kOrderXcds % combos == 0) {
-    return {l * (kOrderXcds / combos) + x / combos, x % combos, combos};
+    return {l * (kOrderXcds / combos) + x / combos, x % combos};
   }
-  return {wg / combos, wg % combos, combos};
+  return {wg / combos, wg % combos};
 }
 // Workgroups that cover `slots` slots of `combos` combos (slots past the last
 // tile find no sequence).
@@ -324,9 +324,10 @@ static int64_t paged_order_grid(int64_t slots, int64_t combos) {
 }
 
 // Compute units, and the workgroups they hold at once, for find_sequence (figures
-// in fa_tiles.h).
+// in fa_tiles.h); slots of a key range where the ranges go one after the other, 0
+// where they go side by side.
 struct PagedOrder {
-  int cus, one_round;
+  int cus, one_round, range_slots;
 };
 
 // Finds the sequence owning slot `tile` in the varlen tile space where
@@ -524,7 +525,7 @@ void fwd_paged_kernel(fa_paged_args a, PagedOrder order) {
 
   int local = 0;
   const int b = find_sequence(a.query_start_loc, a.prefix_kv_lens, a.batch, G, S::BM,
-                              sc.combo_count, order, slot, &local);
+                              a.num_kv_heads, order, slot, &local);
   if (b < 0) return;
   const int qs = a.query_start_loc[b];
   const int qlen = a.query_start_loc[b + 1] - qs;
@@ -546,13 +547,18 @@ void fwd_paged_split_kernel(fa_paged_args a, PagedOrder order, int nsplit, float
                             float* plse) {
   using S = FwdKernelCfg<D, PP>;
   const int G = a.num_heads / a.num_kv_heads;
-  const SlotCombo sc = paged_order(blockIdx.x, a.num_kv_heads * nsplit);
-  const int hk = sc.combo / nsplit, split = sc.combo % nsplit;
-  const int slot = sc.slot;
+  // Ranges of a slot side by side, or (order.range_slots of them each) one range
+  // after the other: see split_range_slots.
+  const bool by_range = order.range_slots > 0;
+  const SlotCombo sc = paged_order(blockIdx.x, by_range ? a.num_kv_heads : a.num_kv_heads * nsplit);
+  const int hk = by_range ? sc.combo : sc.combo / nsplit;
+  const int split = by_range ? sc.slot / order.range_slots : sc.combo % nsplit;
+  const int slot = by_range ? sc.slot % order.range_slots : sc.slot;
+  if (split >= nsplit) return;  // a grid rounded up to whole XCDs
 
   int local = 0;
   const int b = find_sequence(a.query_start_loc, a.prefix_kv_lens, a.batch, G, S::BM,
-                              sc.combo_count, order, slot, &local);
+                              a.num_kv_heads * nsplit, order, slot, &local);
   if (b < 0) return;
   const int qs = a.query_start_loc[b];
   const int qlen = a.query_start_loc[b + 1] - qs;
@@ -744,13 +750,26 @@ static bool paged_few_rows(const fa_paged_args& a, int nsplit) {
   return a.head_dim != 256 || t.wgs * nsplit < device_cu_count() || t.rows > bm * t.seqs;
 }
 
+// Order of a split problem's key ranges.  Side by side, the long tiles of every
+// range go first; but a range ends at a tile's causal limit, so of a long prompt
+// the last range holds the short tiles and the others only whole ones, which
+// then also went last: one range after the other there
+// (kSplitByRangeTokens new tokens a sequence).
+static int split_range_slots(const fa_paged_args& a, int nsplit) {
+  if (nsplit <= 1 || a.num_tokens < tiles::kSplitByRangeTokens * paged_tiles(a).seqs) return 0;
+  return paged_grid_slots(a);
+}
+
 template <class T, int D, bool PP, bool FEW>
 static hipError_t launch_paged_pp(const fa_paged_args& a, int nsplit, void* ws,
                                   hipStream_t st) {
-  const unsigned grid = (unsigned)paged_order_grid(
-      paged_grid_slots(a), (int64_t)a.num_kv_heads * std::max(nsplit, 1));
+  const int64_t slots = paged_grid_slots(a);
+  const int range_slots = split_range_slots(a, nsplit);
+  const unsigned grid = (unsigned)(range_slots > 0
+      ? paged_order_grid(slots * nsplit, a.num_kv_heads)
+      : paged_order_grid(slots, (int64_t)a.num_kv_heads * std::max(nsplit, 1)));
   const int cus = device_cu_count();
-  const PagedOrder order{cus, cus * FwdKernelCfg<D, PP>::WG_PER_CU};
+  const PagedOrder order{cus, cus * FwdKernelCfg<D, PP>::WG_PER_CU, range_slots};
   if (nsplit <= 1) {
     hipLaunchKernelGGL((fwd_paged_kernel<T, D, PP, FEW>), dim3(grid),
                        dim3(FwdKernelCfg<D, PP>::THREADS), 0, st, a, order);

@@ -201,6 +201,15 @@ constexpr int kSplitMinKeys = 4096;
 constexpr int kSplitMinRangeKeys = 1024;
 constexpr int kSplitMaxRangeKeys = 8192;
 constexpr int kMaxSplits = 64;
+// Key ranges one after the other instead of side by side (fa_fwd.hip
+// split_range_slots) from this many new tokens a sequence on (us, side by side / in
+// turn, 2 ranges unless noted): one of 2146 tokens after 2k keys, 16 / 2 heads
+// 136 / 85; one of 1213, D = 256 158 / 106; one of 1051 after 13k, 32 / 8 218 / 189;
+// two of 1517 after 1.5k, 28 / 4 216 / 176; three of 703, 16 / 2 125 / 110; below it,
+// one of 507 after 15k, 28 / 4, D = 64, 6 ranges 112 / 122; three of 344 after 28k,
+// 16 / 16, D = 64, 4 ranges 197 / 221; 12 of 210, 16 / 16, D = 64 159 / 175; 21 of 35
+// after 10k, 28 / 4, 4 ranges 156 / 193.
+constexpr int64_t kSplitByRangeTokens = 512;
 
 // ---- workgroup order of the paged kernels (fa_fwd.hip paged_order,
 // find_sequence).  Up to two rounds of (tile, KV head, key range) workgroups
