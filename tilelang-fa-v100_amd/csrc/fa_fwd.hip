@@ -739,7 +739,8 @@ static PagedTiles paged_tiles(const fa_paged_args& a) {
 // and more than the last rows of a single prompt.  Its workgroups at head_dim
 // 256 have half the bytes in flight of the row-tile core's (one buffer in LDS),
 // so once every CU has one, and with them the memory is busy, they lose
-// (figures at kPagedFewMinKeys), except in batches that are mostly full tiles.
+// (figures at kPagedFewMinKeys), except between tiles of more rows (half a tile's
+// on average).
 static bool paged_few_rows(const fa_paged_args& a, int nsplit) {
   const int64_t lim = int64_t(1) << 24;
   if (a.head_dim > 256 || a.page_size < 16 || a.k_stride[1] >= lim || a.v_stride[1] >= lim)
@@ -747,7 +748,7 @@ static bool paged_few_rows(const fa_paged_args& a, int nsplit) {
   const PagedTiles t = paged_tiles(a);
   const int64_t bm = paged_block_rows(a);
   if (t.rows > tiles::kPagedFewMaxTiles * bm * t.seqs || (t.seqs == 1 && t.rows > 32)) return false;
-  return a.head_dim != 256 || t.wgs * nsplit < device_cu_count() || t.rows > bm * t.seqs;
+  return a.head_dim != 256 || t.wgs * nsplit < device_cu_count() || 2 * t.rows > bm * t.seqs;
 }
 
 // Order of a split problem's key ranges.  Side by side, the long tiles of every

@@ -244,7 +244,8 @@ constexpr int kPagedOrderPairKeys = 1024;
 // 8192 45.5 / 32.3, 288 / 210; 32 (256 workgroups) 48.7 / 49.5, 347 / 381; 64 101 / 105,
 // 682 / 747.  Mixed with chunks, D = 128: 3 sequences, one of a token, 32 / 8 heads, 644
 // rows a sequence, 7k keys 75 / 65; D = 256: 39 of 3-9k keys, 20 of them chunks of 116
-// tokens 767 / 687.
+// tokens 767 / 687; 19 of 8-16k, 16 / 16 heads, 109 rows a sequence 888 / 816; 18, 63
+// rows a sequence 610 / 643.
 constexpr int kPagedFewMinKeys = 384;
 constexpr int kPagedFewMaxTiles = 8;
 
