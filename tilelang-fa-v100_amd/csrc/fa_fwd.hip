@@ -754,10 +754,14 @@ static bool paged_few_rows(const fa_paged_args& a, int nsplit) {
 // Order of a split problem's key ranges.  Side by side, the long tiles of every
 // range go first; but a range ends at a tile's causal limit, so of a long prompt
 // the last range holds the short tiles and the others only whole ones, which
-// then also went last: one range after the other there
-// (kSplitByRangeTokens new tokens a sequence).
+// then also went last: one range after the other there (kSplitByRangeTokens new
+// tokens a sequence, an eighth of a range).
 static int split_range_slots(const fa_paged_args& a, int nsplit) {
-  if (nsplit <= 1 || a.num_tokens < tiles::kSplitByRangeTokens * paged_tiles(a).seqs) return 0;
+  if (nsplit <= 1) return 0;
+  const int64_t seqs = paged_tiles(a).seqs, kv_cap = (int64_t)a.max_blocks * a.page_size;
+  if (a.num_tokens < tiles::kSplitByRangeTokens * seqs ||
+      8 * (int64_t)a.num_tokens * nsplit < kv_cap * seqs)
+    return 0;
   return paged_grid_slots(a);
 }
 
@@ -834,16 +838,34 @@ int paged_num_splits(const fa_paged_args& a) {
   const auto [rows, seqs, wgs] = paged_tiles(a);
   const int64_t kv_cap = (int64_t)a.max_blocks * a.page_size;
   const int cus = device_cu_count();
-  if (kv_cap < tiles::kSplitMinKeys || 2 * wgs >= 3 * cus) return 1;
-  // Below 1.5 workgroups per CU no range is longer than kSplitMaxRangeKeys (a
-  // workgroup's serial length); below one, about one workgroup per CU, or two
-  // where the tiles hold few rows (tiles bound by latency, whose partials are
-  // small); never shorter than kSplitMinRangeKeys (each split adds a partial O
-  // per row to write and merge).
-  int64_t ns = (kv_cap + tiles::kSplitMaxRangeKeys - 1) / tiles::kSplitMaxRangeKeys;
+  if (kv_cap < tiles::kSplitMinKeys) return 1;
+  if (wgs >= cus) {
+    // Every CU has a workgroup.  More ranges only shorten the last round, and
+    // pay for it in partials of every row and a second launch: not for full
+    // tiles.  Two ranges where one-token sequences have the longest tiles,
+    // among chunks, in at most one and a half rounds.  At head_dim 64, whose
+    // CUs hold two workgroups: three for batches of few rows a sequence, up to
+    // four for full tiles after long histories.
+    const bool mixed = a.num_tokens > seqs;
+    const int64_t many = mixed && a.head_dim == 64 ? tiles::kSplitMinKeys : tiles::kSplitMaxRangeKeys;
+    if (kv_cap <= many) return 1;
+    const int bm = paged_block_rows(a);
+    if (a.head_dim == 64) {
+      if (2 * rows <= bm * seqs && wgs < 2 * (int64_t)cus) return 3;
+      if (2 * wgs >= 3 * (int64_t)cus || kv_cap <= 2 * tiles::kSplitMaxRangeKeys) return 1;
+      return (int)std::min<int64_t>(4, (kv_cap + tiles::kSplitMaxRangeKeys - 1) / tiles::kSplitMaxRangeKeys);
+    }
+    const int64_t full = (rows + bm - 1) / bm;
+    return mixed && full <= seqs && 2 * (seqs + full) * a.num_kv_heads <= 3 * (int64_t)cus ? 2 : 1;
+  }
+  // No range is longer than kSplitMaxRangeKeys (a workgroup's serial length);
+  // about one workgroup per CU, or two where the tiles hold few rows (tiles
+  // bound by latency, whose partials are small); never shorter than
+  // kSplitMinRangeKeys (each split adds a partial O per row to write and merge).
   const bool few = rows <= 32 * seqs;
   const int64_t want = few ? 2 * cus : cus;
-  if (wgs < cus) ns = std::max<int64_t>(ns, (want + wgs - 1) / wgs);
+  int64_t ns = std::max<int64_t>((kv_cap + tiles::kSplitMaxRangeKeys - 1) / tiles::kSplitMaxRangeKeys,
+                                 (want + wgs - 1) / wgs);
   ns = std::min<int64_t>(ns, kv_cap / tiles::kSplitMinRangeKeys);
   return (int)std::max<int64_t>(1, std::min<int64_t>(ns, kMaxPagedSplits));
 }

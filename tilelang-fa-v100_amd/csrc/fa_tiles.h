@@ -179,12 +179,12 @@ constexpr int kDecTilesInFlight = 2;
 // 8 TB/s; 64 x 16k keys at D = 128, pages of 1-8 keys: 65-67%.
 constexpr int kDecChunkElems = 32768;
 
-// ---- split-KV paged prefill (fa_fwd.hip paged_num_splits): no split when
-// the tiles (at least one per sequence) give 1.5 workgroups per CU or the
-// block table holds fewer than kSplitMinKeys keys; otherwise
-// ceil(keys / kSplitMaxRangeKeys) ranges, and below one workgroup per CU at
-// least ceil(CUs / workgroups) (twice that for tiles of few rows), but none
-// shorter than kSplitMinRangeKeys and at most kMaxSplits.
+// ---- split-KV paged prefill (fa_fwd.hip paged_num_splits): no split when the
+// block table holds fewer than kSplitMinKeys keys; with fewer workgroups (row
+// tiles, at least one per sequence, x KV heads) than CUs
+// max(ceil(keys / kSplitMaxRangeKeys), ceil(CUs / workgroups)) ranges (twice the
+// CUs for tiles of few rows), but none shorter than kSplitMinRangeKeys and at
+// most kMaxSplits; from one workgroup per CU on one range, or two (below).
 // Evidence (2 sequences, 32 / 8 heads, D = 128, time per call in ms for
 // 1 / 4 / 8 / 16 splits): 32k-key prefix + 128 tokens 0.955 / 0.277 / 0.171 /
 // 0.192 (this rule: 8); 16k + 128: 0.487 / 0.153 / 0.104 / 0.128 (8);
@@ -197,6 +197,19 @@ constexpr int kDecChunkElems = 32768;
 // 2-16k keys 198 / 144 / 120 / 134 (4; was 16); 47 of them with a 512-token
 // chunk, 64 heads 167 / 198 / 229 / 302 (1; was 2); 30 with two chunks, table
 // of 16k keys 162 / 150 / 187 / 243 (2; was 3).
+// From one workgroup per CU on (us for 1 / 2 / 3 ranges).  Full tiles: 16 chunks of
+// 198-396 tokens, 16 / 16 heads 173 / 213 / 223; 6 of 352-704 after 3-12k keys, 32 / 8
+// 437 / 458 / 458; 8 of 457-914, D = 256 190 / 218 / 225; 3 of 1378 after 6-25k, 16 / 2
+// 608 / 657 / 636; none is faster split.  One-token sequences alone, 1-8k keys, D = 128:
+// 20 of 16 / 16 heads 45 / 55 / 57 (1.1k keys), 142 / 130 / 127 (4.7k); 43 of 32 / 8
+// 149 / 156 / 164.  With a chunk or two among them, tiles up to 1.5 per CU: 37, 32 / 8
+// 192 / 137 / 138; 20, 16 / 16 172 / 140 / 136; 32, 32 / 8 157 / 119 / 126; 16 of 1.5k
+// keys in a table of 4.5k 42 / 49 / 53; D = 256: 34, 32 / 8 525 / 435 / 427.  Above: 42,
+// 64 / 8 (576) 312 / 378 / 389.  D = 64, two workgroups a CU: 35, 64 / 8, table of 4.1k 85 /
+// 68 / 59; one-token sequences alone, 18 of 5.3k, 16 / 16 121 / 99 / 88; 46 of 7.8k, 64 / 8
+// 187 / 172 / 165; 42 of 1.2k, 64 / 8 in a table of 32k 31 / 39 / 37; more rows, 52 and 26
+// chunks, 32 / 8 (624 tiles) 68 / 87 / 92; full tiles, 7 chunks of 216 after 8-32k, 28 / 4
+// 497, 396 in four ranges, 20 of 65 after 1-4k, 32 / 8 79 / 86.
 constexpr int kSplitMinKeys = 4096;
 constexpr int kSplitMinRangeKeys = 1024;
 constexpr int kSplitMaxRangeKeys = 8192;
@@ -205,8 +218,9 @@ constexpr int kMaxSplits = 64;
 // split_range_slots) from this many new tokens a sequence on (us, side by side / in
 // turn, 2 ranges unless noted): one of 2146 tokens after 2k keys, 16 / 2 heads
 // 136 / 85; one of 1213, D = 256 158 / 106; one of 1051 after 13k, 32 / 8 218 / 189;
-// two of 1517 after 1.5k, 28 / 4 216 / 176; three of 703, 16 / 2 125 / 110; below it,
-// one of 507 after 15k, 28 / 4, D = 64, 6 ranges 112 / 122; three of 344 after 28k,
+// two of 1517 after 1.5k, 28 / 4 216 / 176; three of 703, 16 / 2 125 / 110; with fewer or
+// in longer ranges, two of 808 after 5-22k, 16 / 2, 3 ranges 263 / 292; seven of 579 after
+// 7-29k, 4 ranges 600 / 656; one of 507 after 15k, 28 / 4, D = 64, 6 112 / 122; three of 344 after 28k,
 // 16 / 16, D = 64, 4 ranges 197 / 221; 12 of 210, 16 / 16, D = 64 159 / 175; 21 of 35
 // after 10k, 28 / 4, 4 ranges 156 / 193.
 constexpr int64_t kSplitByRangeTokens = 512;
