@@ -33,7 +33,7 @@ CASES = [
     ([1, 8, 9, 1, 1, 1], [383, 384, 385, 415, 513, 767], 16, 4, 128, 16, F16, True, -1, -1, 1),
     ([1, 1, 8, 2, 1], [1151, 1152, 1154, 1249, 1700], 16, 4, 128, 32, BF16, True, -1, -1, 3),
     ([1, 1, 8, 1], [383, 384, 417, 2051], 8, 2, 64, 16, F16, True, -1, -1, 1),
-    ([1, 3, 1], [384, 497, 777], 16, 2, 256, 16, F16, True, -1, -1, 1),
+    ([1, 3, 1, 1], [384, 497, 777, 128], 16, 2, 256, 16, F16, True, -1, -1, 1),
     ([1] * 20, [384 + 5 * i for i in range(20)], 16, 16, 256, 16, F16, True, -1, -1, 1),  # > CUs
     ([1, 1, 900], [900, 2000, 1000], 64, 8, 128, 16, F16, True, -1, -1, 1),  # mostly full tiles
 ]

@@ -491,7 +491,7 @@ __device__ __forceinline__ void run_paged_tile(const fa_paged_args& a, int rows,
     constexpr int kSplitLds = FwdSplitShape<D, NW>::LDS;
     constexpr int kLds = kSplitLds > C::LDS_BYTES ? kSplitLds : C::LDS_BYTES;
     __shared__ __attribute__((aligned(16))) char smem[kLds];
-    if (rows <= 32 && keys() >= tiles::kPagedFewMinKeys) {
+    if (rows <= 32 && keys() >= (D == 256 ? tiles::kPagedFewMinKeys256 : tiles::kPagedFewMinKeys)) {
       const auto* ap = kernel_args<fa_paged_args>();
       Prob P;
       setup(*ap, P);

@@ -249,7 +249,7 @@ constexpr int kPagedOrderPairKeys = 1024;
 
 // ---- paged tiles of at most 32 rows (fa_fwd.hip run_paged_tile, paged_few_rows):
 // their keys are split over the workgroup's waves from kPagedFewMinKeys keys (of
-// the tile's range) on, in batches of at most kPagedFewMaxTiles full tiles per
+// the tile's range; head_dim 256 kPagedFewMinKeys256) on, in batches of at most kPagedFewMaxTiles full tiles per
 // sequence.  Evidence (us, one-token sequences, row-tile / key-split core, one
 // range): D = 128, 32 / 8 heads, 16 sequences of 512 / 2048 / 8192 keys 19.7 / 18.1,
 // 48.7 / 31.1, 190 / 125; 128 of 128 / 256 / 512 / 2048 keys 33.2 / 38.5, 45.1 / 47.0,
@@ -261,6 +261,7 @@ constexpr int kPagedOrderPairKeys = 1024;
 // tokens 767 / 687; 19 of 8-16k, 16 / 16 heads, 109 rows a sequence 888 / 816; 18, 63
 // rows a sequence 610 / 643.
 constexpr int kPagedFewMinKeys = 384;
+constexpr int kPagedFewMinKeys256 = 128;  // 16 sequences of 128 / 256 keys 15.3 / 14.6, 20.0 / 16.8
 constexpr int kPagedFewMaxTiles = 8;
 
 }  // namespace tiles
