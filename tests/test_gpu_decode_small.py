@@ -37,3 +37,17 @@ def test_small_batches(case):
     bt = torch.cat([bt, bt.new_full((bt.shape[0], width - bt.shape[1]), -1)], 1)
     print(f"case {case}", flush=True)
     check((q, kc, vc, bt, sl, page))
+
+
+@pytest.mark.parametrize("batch,Hq,Hkv,D,table", [(72, 32, 8, 128, 0), (72, 32, 8, 128, 32768),
+                                                  (130, 16, 2, 512, 0), (64, 32, 32, 64, 0),
+                                                  (63, 32, 4, 256, 8192)])
+def test_many_rows(batch, Hq, Hkv, D, table):
+    """Eight (sequence, head) rows a CU on either side: the one-wave merge, with one partial, many
+    and none; batches of more than 64 lengths."""
+    lens = [(37 * i) % 700 for i in range(batch - 2)] + [3000, 1025]
+    q, kc, vc, bt, sl, page = make_case(53, lens, Hq, Hkv, D, page=16, dtype=torch.float16)
+    width = max(bt.shape[1], table // page)
+    bt = torch.cat([bt, bt.new_full((bt.shape[0], width - bt.shape[1]), -1)], 1)
+    print(f"case {batch} {Hq}/{Hkv} D{D}", flush=True)
+    check((q, kc, vc, bt, sl, page))

@@ -206,18 +206,19 @@ __global__ __launch_bounds__(256, 2) void decode_split_kernel(fa_decode_args a,
   }
 }
 
-// One workgroup of kCombineWaves waves per (sequence, query head): merge the
-// chunk partials with weights exp2(lse_c - max), computed lane-parallel, then
-// an unrolled weighted sum.  Bound by the latency of a wave's chain of partial
-// loads (a long sequence has up to 128 of them), so the waves take the
-// partials in turn and their sums meet in LDS.
-constexpr int kCombineWaves = 4;
-template <class T, int D>
-__global__ __launch_bounds__(64 * kCombineWaves) void decode_combine_kernel(fa_decode_args a,
-                                                                          DecodeWs ws) {
+// One workgroup of NW waves per (sequence, query head): merge the chunk partials
+// with weights exp2(lse_c - max), computed lane-parallel, then an unrolled
+// weighted sum.  Bound by the latency of a wave's chain of partial loads (a long
+// sequence has up to 128 of them), so with few rows four waves take the
+// partials in turn and their sums meet in LDS; from eight rows per CU on the
+// rows themselves hide it and the extra waves only cost their start (us per
+// call, one / four waves: 4 sequences of 0.5-8k keys, 32 heads 25 / 22; 109 of
+// 33-534, 64 heads, D = 512 159 / 170; 72 of 0.2-2.4k, 64 heads, D = 128 74.5 / 77).
+constexpr int kCombineWaves = 4, kCombineRowsPerCU = 8;
+template <class T, int D, int NW>
+__global__ __launch_bounds__(64 * NW) void decode_combine_kernel(fa_decode_args a, DecodeWs ws) {
   const int CH = ws.split_dev ? *ws.split_dev : ws.split;
   constexpr int NP = (D + 127) / 128;  // d pairs per lane: 2*lane + 128*k
-  constexpr int NW = kCombineWaves;
   __shared__ float wts[NW][64];
   __shared__ __attribute__((aligned(8))) float part[NW][D];
   const int hq = blockIdx.x % a.num_heads;
@@ -360,8 +361,13 @@ int device_cu_count() {
 
 template <class T, int D>
 static hipError_t launch_combine(const fa_decode_args& a, DecodeWs ws, hipStream_t st) {
-  hipLaunchKernelGGL((decode_combine_kernel<T, D>), dim3((unsigned)(a.batch * a.num_heads)),
-                     dim3(64 * kCombineWaves), 0, st, a, ws);
+  const int64_t rows = (int64_t)a.batch * a.num_heads;
+  if (rows >= kCombineRowsPerCU * (int64_t)device_cu_count())
+    hipLaunchKernelGGL((decode_combine_kernel<T, D, 1>), dim3((unsigned)rows), dim3(64), 0, st, a,
+                       ws);
+  else
+    hipLaunchKernelGGL((decode_combine_kernel<T, D, kCombineWaves>), dim3((unsigned)rows),
+                       dim3(64 * kCombineWaves), 0, st, a, ws);
   return hipGetLastError();
 }
 

@@ -244,30 +244,36 @@ void decode_stream_kernel(fa_decode_args a, DecodeWsS ws) {
   __shared__ int split_sh;
   if (wv == 0) {
     int split = ws.split;
+    // Lengths of the sequences b0 .. b0 + 63, one per lane; the first 64 are
+    // read once (every read is a trip to the L2 that the whole workgroup waits
+    // for).
+    auto read_len = [&](int b0) {
+      return b0 + lane < B ? max(0, min(a.seq_lens[b0 + lane], cap)) : 0;
+    };
+    const int len0 = read_len(0);
+    auto len_of = [&](int b0) { return b0 == 0 ? len0 : read_len(b0); };
     // Items per head slot at a split of n keys.
     auto units = [&](int n) {
       int sum = 0;
-      for (int b0 = 0; b0 < B; b0 += 64) {
-        const int b = b0 + lane;
-        const int len = b < B ? max(0, min(a.seq_lens[b], cap)) : 0;
-        sum += wave_total((len + n - 1) / n);
-      }
+      for (int b0 = 0; b0 < B; b0 += 64) sum += wave_total((len_of(b0) + n - 1) / n);
       return sum;
     };
-    if ((int64_t)B * HG * 2 < ws.waves) {
-      // Few sequences: block tables are often as wide as the longest context
-      // the model takes, so the launcher's split can be far too long.
+    const int64_t first = (int64_t)units(split) * HG;
+    if (2 * first < ws.waves) {
+      // Few items: block tables are often as wide as the longest context the
+      // model takes, so the launcher's split can be far too long.
       int longest = 0;
-      for (int b0 = 0; b0 < B; b0 += 64)
-        longest = max(longest, b0 + lane < B ? max(0, min(a.seq_lens[b0 + lane], cap)) : 0);
-#pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) longest = max(longest, __shfl_xor(longest, o));
-      while (split > tiles::kDecSplitKeysMin &&
-             (longest + split / 2 - 1) / (split / 2) <= ws.nsplit &&  // the partials fit
-             (int64_t)units(split) * HG * 2 < ws.waves)
+      for (int b0 = 0; b0 < B; b0 += 64) longest = max(longest, wave_max_nonneg(len_of(b0)));
+      do {
+        if (split <= tiles::kDecSplitKeysMin ||
+            (longest + split / 2 - 1) / (split / 2) > ws.nsplit)  // the partials fit
+          break;
         split /= 2;
+      } while ((int64_t)units(split) * HG * 2 < ws.waves);
+    } else if (first >= tiles::kDecItemsPerWave * (int64_t)ws.waves &&
+               (int64_t)units(2 * split) * HG >= tiles::kDecItemsPerWave * (int64_t)ws.waves) {
+      split *= 2;
     }
-    if ((int64_t)units(2 * split) * HG >= (int64_t)tiles::kDecItemsPerWave * ws.waves) split *= 2;
     if (lane == 0) {
       split_sh = split;
       if (blockIdx.x == 0) *ws.split_out = split;
@@ -275,12 +281,7 @@ void decode_stream_kernel(fa_decode_args a, DecodeWsS ws) {
     int base = 0;
     for (int b0 = 0; b0 < B; b0 += 64) {
       const int b = b0 + lane;
-      int cnt = 0;
-      if (b < B) {
-        const int len = max(0, min(a.seq_lens[b], cap));
-        cnt = (len + split - 1) / split;
-      }
-      const int incl = wave_scan(cnt);
+      const int incl = wave_scan((len_of(b0) + split - 1) / split);
       if (b < B) pfx[b + 1] = base + incl;
       base += __builtin_amdgcn_readlane(incl, 63);
     }
