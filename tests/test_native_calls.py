@@ -1,9 +1,14 @@
 """The native call marshalling against the Python path it stands in for.
 
-On the CPU: what is not the plain case is handed back (None) before any work.
+On the CPU: what is not the plain case is handed back (None) before any work,
+and so is every call where the extension is not built for this torch.
 On the GPU: every form a caller may pass gives the same bits whether the native
 path takes it or not, and mistakes raise the same exception either way.
 """
+import sys
+import types
+import warnings
+
 import pytest
 import torch
 
@@ -28,6 +33,30 @@ def test_cpu_tensors_and_foreign_objects_are_handed_back():
     assert _native.dense_forward(t, t, t, 0.1, True, (-1, -1), True) is None
     with pytest.raises(TypeError):
         m.bind(1)
+
+
+@pytest.mark.parametrize("found", [None, types.ModuleType("stale"),
+                                   types.SimpleNamespace(torch_version="1.0")],
+                         ids=["none", "no version", "another torch"])
+def test_without_the_extension_python_takes_the_calls(found, monkeypatch):
+    """One warning, then every call is handed back; load() itself still says what is missing."""
+    monkeypatch.setattr(_native, "_module", None)
+    monkeypatch.setattr(_native, "_missing", False)
+    monkeypatch.setitem(sys.modules, "tilelang_fa_v100._fa_torch", found)
+    monkeypatch.delattr(fa, "_fa_torch", raising=False)
+    if found is not None:
+        monkeypatch.setattr(fa, "_fa_torch", found, raising=False)
+    with pytest.raises(RuntimeError, match="not built for this torch"):
+        _native.load()
+    device = types.SimpleNamespace(is_cuda=True)
+    monkeypatch.setattr(_native, "torch", types.SimpleNamespace(
+        Tensor=types.SimpleNamespace, __version__=torch.__version__))
+    with pytest.warns(RuntimeWarning, match="marshalled in Python"):
+        assert _native.decode(device) is None
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert _native.dense_forward(device, device, device, 0.1, True, (-1, -1), True) is None
+        assert _native.cache_write(device) is None
 
 
 def _dense(**over):

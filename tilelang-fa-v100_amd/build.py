@@ -80,6 +80,15 @@ def _run(cmd: list[str], verbose: bool) -> None:
         print(res.stdout + res.stderr, flush=True)
 
 
+def _rocm_clang() -> str:
+    """The host C++ compiler that hipcc itself runs."""
+    for name in ("lib/llvm/bin/clang++", "llvm/bin/clang++"):
+        path = os.path.join(os.path.dirname(os.path.dirname(hipcc())), name)
+        if os.path.exists(path):
+            return path
+    raise RuntimeError("no host C++ compiler found (set CXX)")
+
+
 def _ext_command() -> list[str]:
     """Host-only C++ against torch's headers; it gets the library's entry
     points as addresses, so it links neither libfa355.so nor the HIP runtime."""
@@ -88,14 +97,13 @@ def _ext_command() -> list[str]:
     import torch
     from torch.utils import cpp_extension
 
-    cxx = os.environ.get("CXX") or shutil.which("g++") or shutil.which("c++")
-    if not cxx:
-        raise RuntimeError("no host C++ compiler found (set CXX)")
+    cxx = os.environ.get("CXX") or shutil.which("g++") or shutil.which("c++") or _rocm_clang()
     inc = [f"-I{p}" for p in (*cpp_extension.include_paths(), sysconfig.get_paths()["include"],
                               INCLUDE)]
     libs = [f"-L{p}" for p in cpp_extension.library_paths()]
     return [cxx, "-O2", "-std=c++17", "-fPIC", "-shared",
-            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *inc,
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            f'-DFA_TORCH_VERSION="{torch.__version__}"', *inc,
             os.path.join(CSRC, "fa_torch.cpp"), "-o", EXT + ".tmp", *libs,
             "-ltorch_python", "-ltorch_cpu", "-lc10"]
 

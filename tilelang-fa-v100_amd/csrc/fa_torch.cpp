@@ -404,4 +404,13 @@ PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_fa_torch", nullptr, -1, metho
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__fa_torch(void) { return PyModule_Create(&module_def); }
+// FA_TORCH_VERSION: the torch whose headers this was compiled against; another
+// one's tensors may be laid out differently, so the loader compares it.
+PyMODINIT_FUNC PyInit__fa_torch(void) {
+  PyObject* m = PyModule_Create(&module_def);
+  if (m && PyModule_AddStringConstant(m, "torch_version", FA_TORCH_VERSION) < 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

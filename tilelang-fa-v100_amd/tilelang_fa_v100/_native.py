@@ -3,12 +3,15 @@
 Each function returns the entry point's result, raises what the library's
 status says, or returns None when the call is not the plain case (CPU or
 foreign-device tensors, subclasses, conversions or copies needed, mistakes):
-the caller's Python path then takes it, with its checks and messages.
+the caller's Python path then takes it, with its checks and messages.  The
+same where the extension is not built for this torch: every call then goes
+through ctypes to the same kernels, after one warning.
 """
 from __future__ import annotations
 
 import ctypes
 import threading
+import warnings
 
 import torch
 
@@ -19,10 +22,12 @@ _ENTRIES = ("fa_fwd", "fa_decode_workspace_bytes", "fa_paged_decode",
             "fa_paged_prefill_splitkv", "fa_reshape_and_cache")
 _lock = threading.Lock()
 _module = None
+_missing = False  # load() failed: the Python path takes every call
 
 
 def load():
-    """The extension module, bound to the library's entry points."""
+    """The extension module, bound to the library's entry points; RuntimeError where it is not
+    built for this torch."""
     global _module
     if _module is None:
         lib = _lib.load()
@@ -30,9 +35,12 @@ def load():
             if _module is None:
                 try:
                     from . import _fa_torch
+                    built = getattr(_fa_torch, "torch_version", None)
+                    if built != torch.__version__:
+                        raise ImportError(f"built for torch {built}")
                 except ImportError as e:
                     raise RuntimeError(
-                        "_fa_torch is not built for this torch; run "
+                        f"_fa_torch is not built for this torch ({e}); run "
                         "`python tilelang-fa-v100_amd/build.py` (or __graft_entry__.build())"
                     ) from e
                 _fa_torch.bind(*(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value
@@ -41,11 +49,29 @@ def load():
     return _module
 
 
+def _extension():
+    """load(), or None with one warning."""
+    global _missing
+    _lib.load()  # the kernels themselves: an error for every call
+    try:
+        return load()
+    except RuntimeError as e:
+        with _lock:
+            first, _missing = not _missing, True
+        if first:
+            warnings.warn(f"{e}; calls are marshalled in Python (several us more each)",
+                          RuntimeWarning, stacklevel=2)
+        return None
+
+
 def _run(name, what, first, args):
-    if not (isinstance(first, torch.Tensor) and first.is_cuda):
+    if _missing or not (isinstance(first, torch.Tensor) and first.is_cuda):
+        return None
+    module = _module or _extension()
+    if module is None:
         return None
     device = torch._C._cuda_getDevice()
-    r = getattr(_module or load(), name)(*args, device, torch._C._cuda_getCurrentRawStream(device))
+    r = getattr(module, name)(*args, device, torch._C._cuda_getCurrentRawStream(device))
     if type(r) is int:
         _lib.check(r, what)
     return r
