@@ -3,7 +3,8 @@
 On the CPU: what is not the plain case is handed back (None) before any work,
 and so is every call where the extension is not built for this torch.
 On the GPU: every form a caller may pass gives the same bits whether the native
-path takes it or not, and mistakes raise the same exception either way.
+path takes it or not, and mistakes raise the same exception either way; the
+native path takes exactly the forms it is for.
 """
 import sys
 import types
@@ -163,6 +164,14 @@ FORMS = {
 }
 
 
+# Forms the native path takes; it hands back all others, and an `out` argument
+# is not put to it.
+TAKEN = {"dense plain", "dense causal int", "dense window", "dense scale int", "dense lse",
+         "dense strided", "dense [B, H, S, D] storage", "dense expanded", "dense one row",
+         "dense parameter", "decode plain", "decode heads given", "paged plain",
+         "paged not causal", "paged windows", "cache plain", "cache strided"}
+
+
 def _outcome(call, make):
     try:
         r = call(make())
@@ -177,7 +186,19 @@ def _outcome(call, make):
 def test_native_and_python_paths_agree(form, monkeypatch):
     call, make = FORMS[form]
     print(f"form {form}", flush=True)
+    taken = []
+
+    def recorded(f):
+        def g(*a, **k):
+            r = f(*a, **k)
+            taken.append(r is not None)
+            return r
+        return g
+
+    for name in NAMES:
+        monkeypatch.setattr(_native, name, recorded(getattr(_native, name)))
     native = _outcome(call, make)
+    assert taken == ([] if form == "paged out" else [form in TAKEN])
     for name in NAMES:
         monkeypatch.setattr(_native, name, lambda *a, **k: None)
     python = _outcome(call, make)
