@@ -102,8 +102,8 @@ int fa_fwd(const fa_fwd_args* args, void* stream);
  * dS tiles from which dq is formed (2 bytes per (query, key) pair the mask
  * lets through, up to 4 GiB); fa_bwd_workspace_bytes gives that size.  A
  * workspace of at least fa_bwd_min_workspace_bytes (the statistics only)
- * selects the path that recomputes S and dP for dq instead; both paths are
- * deterministic. */
+ * selects the path that recomputes S and dP for dq instead, and one of
+ * fa_bwd_preferred_workspace_bytes the fastest; every path is deterministic. */
 typedef struct fa_bwd_args {
   const void* q;
   const void* k;
@@ -134,9 +134,12 @@ typedef struct fa_bwd_args {
   int32_t deterministic; /* accepted and ignored, as in the reference
                           * (interface.py:16-17): the backward has no atomics
                           * (each dq row is summed by one wave in a fixed
-                          * order), so dq, dk and dv always repeat bit for bit,
-                          * like the reference's kernels
-                          * (_kernels_backward.py:10-85,88-176) */
+                          * order), so dq, dk and dv repeat bit for bit, like
+                          * the reference's kernels
+                          * (_kernels_backward.py:10-85,88-176), for the same
+                          * path: the workspace's size selects it (below), and
+                          * the fp32 sums of dq, or of dk and dv, have another
+                          * order on another path */
   int32_t has_window;    /* as in fa_fwd_args */
   int32_t window_left;
   int32_t window_right;

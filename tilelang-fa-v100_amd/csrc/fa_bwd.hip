@@ -25,8 +25,9 @@
 // (_kernels_backward.py:74,160), so dS has fp16's full range.
 //   bwd_main_mfma_kernel  dK / dV (fa_bwd_mfma.h); for small grids as several
 //                       pieces per key tile, summed by bwd_reduce_kernel.
-// At head_dim 128 / 256 with causal or full attention and a workspace of
-// bwd_workspace_bytes, the order is instead bwd_stats_kernel (the row
+// At head_dim 128 / 256 with a workspace of bwd_workspace_bytes (causal or full
+// attention) or bwd_preferred_workspace_bytes (window bands too), the order is
+// instead bwd_stats_kernel (the row
 // statistics), bwd_main_mfma_kernel<..., DS = true> (dK / dV, storing its dS
 // tiles) and bwd_dq_ds_kernel (dQ = dS K from them), fa_bwd_ds.h.
 #include "fa_bwd_dq.h"
@@ -155,8 +156,8 @@ size_t bwd_preferred_workspace_bytes(const fa_bwd_args& a) {
 }
 
 // Key-stationary dK / dV kernel for one mask mode; with ds, also stores the
-// dS tiles (head_dim 128 / 256, causal or full attention); with pieces > 1
-// (those cases and head_dim 64), as that many pieces per workgroup whose sums
+// dS tiles (head_dim 128 / 256); with pieces > 1 (causal or full attention; at
+// head_dim 128 / 256 only with ds), as that many pieces per workgroup whose sums
 // land in `part`, then their reduction.
 template <class T, int D, int MODE, bool DS, bool SPLIT>
 static void launch_main(const fa_bwd_args& a, const float* stats, uint16_t* ds, float* part,

@@ -167,8 +167,8 @@ void bwd_dq_kernel(fa_bwd_args a, float* stats) {
   // block blk holds row RPB blk + l / CPR, stored chunk l % CPR (logical
   // chunk (l % CPR) ^ swz(row)).  The rows go through buffer resources based
   // at the wave's first row: the lane's byte offset is fixed for the whole
-  // loop (below 8 rows, so 32 bits hold it for any sequence stride below
-  // 2^26), and rows at or past the last key read as zero (their scores are
+  // loop (at most WR <= 16 rows, so 32 bits hold it for any sequence stride
+  // below 2^26), and rows at or past the last key read as zero (their scores are
   // masked).
   constexpr int WR = S::RPB * S::BPW;
   const uint16_t* kg = static_cast<const uint16_t*>(a.k) + b * a.k_stride[0] + hk * a.k_stride[2];

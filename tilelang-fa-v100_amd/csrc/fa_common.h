@@ -224,17 +224,6 @@ __device__ __forceinline__ void st8(void* p, u32x2 v) {
 // causal is wr = 0), off = Sk - Sq.  Row / key bounds are checked separately.
 struct Band {
   int off, wl, wr;
-  // Some pair with i in [i0, i1] and j in [j0, j1] is inside the band.
-  __device__ bool any(int i0, int i1, int j0, int j1) const {
-    return (wr < 0 || j0 <= i1 + off + wr) && (wl < 0 || j1 >= i0 + off - wl);
-  }
-  // Every such pair is inside the band.
-  __device__ bool all(int i0, int i1, int j0, int j1) const {
-    return (wr < 0 || j1 <= i0 + off + wr) && (wl < 0 || j0 >= i1 + off - wl);
-  }
-  __device__ bool in(int i, int j) const {
-    return (wr < 0 || j <= i + off + wr) && (wl < 0 || j >= i + off - wl);
-  }
   // Query rows [first, end) that see any key in [j0, j1], clipped to [0, sq).
   __device__ int first_row(int j0) const { return wr >= 0 ? max(0, j0 - off - wr) : 0; }
   __device__ int end_row(int j1, int sq) const {

@@ -81,8 +81,8 @@ struct FwdKernelCfg<128, PP> {
   static constexpr int LDS_BYTES = FwdShapeD128::LDS_BYTES;
 };
 
-// LDS: one array for the 4-wave core; four distinct arrays for the D = 128
-// cores (see attn_fwd_tile_d128).  PP: the ping-pong D = 128 core, which
+// LDS: one array for the 4-wave core; four regions for the D = 128 cores (see
+// attn_fwd_tiles_d128).  PP: the ping-pong D = 128 core, which
 // needs 16 consecutive keys at a fixed row stride (dense rows, or pages of
 // at least 16 keys) with row strides below 2^24 elements; otherwise the
 // one-phase core.

@@ -69,10 +69,10 @@ __device__ __forceinline__ void wait_vmem() { __builtin_amdgcn_s_waitcnt(0x0F70)
 // tile between two barriers), used for paged problems whose pages hold fewer
 // than 16 keys: their K / V rows need a block-table read each (the ping-pong
 // schedule below takes 16-key runs at a fixed stride).
-// k0/v0 and k1/v1 are four distinct __shared__ arrays of TILEB bytes.  The
-// loop is unrolled by two so that every LDS read names one array pair while
-// the DMA of the next tile targets the other; the compiler can then see that
-// the reads do not depend on the outstanding DMA and does not wait for it.
+// k0/v0 and k1/v1 are four LDS regions of TILEB bytes that do not overlap.  The
+// loop is unrolled by two so that every LDS read names one pair while the DMA
+// of the next tile targets the other; the compiler can then see that the reads
+// do not depend on the outstanding DMA and does not wait for it.
 template <class T, class Prob>
 __device__ __forceinline__ void attn_fwd_tile_d128_plain(const Prob& P, int row0, float scale,
                                                    char* k0, char* v0, char* k1, char* v1) {
@@ -246,10 +246,12 @@ __device__ __forceinline__ void attn_fwd_tile_d128_plain(const Prob& P, int row0
 
 
 // Ping-pong schedule, used for row-strided (dense) problems.
-// k0/v0 and k1/v1 are four distinct __shared__ arrays of TILEB bytes.  The
-// loop is unrolled by two so that every LDS read names one array pair while
-// the DMA of the next tile targets the other; the compiler can then see that
-// the reads do not depend on the outstanding DMA and does not wait for it.
+// k0/v0 and k1/v1 are four LDS regions of TILEB bytes that do not overlap: arrays
+// of their own, or (run_paged_tile) quarters of one that another core shares.
+// The loop is unrolled by two so that every LDS read names one pair while the
+// DMA of the next tile targets the other; the compiler can then see that the
+// reads do not depend on the outstanding DMA and does not wait for it (one
+// vmcnt(0) a barrier in the compiled loop, in both forms).
 //
 // attn_fwd_tiles_d128 runs a sequence of row tiles on one workgroup:
 // next(P, row0) rewrites the problem and first row for the next tile and

@@ -20,8 +20,9 @@ hipError_t launch_fwd(const fa_fwd_args& a, hipStream_t st);
 // tiles::kBwdDsMaxBytes), else the row statistics only.
 // bwd_min_workspace_bytes: the row statistics (the recompute path).
 size_t bwd_workspace_bytes(const fa_bwd_args& a);
-// bwd_preferred_workspace_bytes: bwd_workspace_bytes plus, where the dK / dV
-// grid is small, the fp32 partials of its split over query tiles.
+// bwd_preferred_workspace_bytes: that plus a window band's dS tiles (head_dim
+// 128 or 256), or, where the dK / dV grid is small, the fp32 partials of its
+// split over query tiles.
 size_t bwd_min_workspace_bytes(const fa_bwd_args& a);
 size_t bwd_preferred_workspace_bytes(const fa_bwd_args& a);
 hipError_t launch_bwd(const fa_bwd_args& a, void* ws, size_t ws_bytes, hipStream_t st);

@@ -102,7 +102,7 @@ def bwd_args(q, k, v, out, dout, lse, dq, dk, dv, softmax_scale, causal, determi
 
 # ---- backward workspace policy
 #
-# fa_bwd runs one of two paths, chosen by the workspace it is given:
+# What fa_bwd runs is chosen by the workspace it is given:
 #  * fa_bwd_min_workspace_bytes: the row statistics only (8 bytes per query
 #    row and head); dQ recomputes S and dP, like the reference's dQ kernel.
 #    This is the memory footprint of the reference's tilelang_backward
@@ -112,9 +112,15 @@ def bwd_args(q, k, v, out, dout, lse, dq, dk, dv, softmax_scale, causal, determi
 #    (query, key) pair: 268 MB at [4, 2048, 16, 128], 2.15 GB at
 #    [2, 8192, 16, 128]); dQ then costs one product per tile pair instead of
 #    three.
-# The dS path is taken while its workspace fits the limit below, and the
-# recompute path whenever it does not or its allocation fails, so the
-# backward never needs more memory than the reference's.
+#  * fa_bwd_preferred_workspace_bytes, where larger: the same for window bands
+#    (dS tiles of the band's width), or the fp32 partials of a dK / dV kernel
+#    that small grids cut into pieces (any head_dim).
+# The largest that fits the limit below is taken, and the recompute path
+# whenever none does or the allocation fails, so the backward never needs more
+# memory than the reference's.  Gradients repeat bit for bit for one workspace
+# size: dq differs in rounding between recomputing and the dS tiles, dk and dv
+# between whole and cut dK / dV kernels.  With plenty of free memory, or with a
+# limit set, every call of a shape takes the same one.
 
 WORKSPACE_LIMIT_ENV = "TILELANG_FA_BWD_WORKSPACE_LIMIT"
 # Default limit: this share of the memory the device can still hand out
