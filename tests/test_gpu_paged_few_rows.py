@@ -76,10 +76,14 @@ def test_tile_orders_cover_every_tile(q_lens, heads):
     ([1, 2, 129, 64, 0, 300] * 10, 300, 4, 64),   # 60 sequences, 320 workgroups: tiles by reach
     ([200, 1, 370, 0, 129, 300] * 2, 0, 50, 64),  # no histories, 700 workgroups: tiles by reach
     ([1100, 300, 0, 700], 0, 32, 128),            # no histories, 320 workgroups: tiles by reach
+    ([1100, 300, 0, 700], 0, 60, 128),            # 600, XCDs share heads: tiles by reach
+    ([1100, 300, 0, 700], 0, 76, 128),            # 760, as above: just below three rounds
+    ([1100, 300, 0, 700], 0, 78, 128),            # 780: sequences in their own order
     ([1100, 300, 0, 700], 0, 32, 256),            # 544, one a CU: sequences in their own order
     ([500, 0, 530], 0, 66, 128),                  # two short prompts: no search
     ([500, 0, 530], 100, 66, 128),                # two histories
-], ids=["by-sequence-reach", "by-reach", "two-rounds-d64", "two-rounds-d128", "own-order-d256",
+], ids=["by-sequence-reach", "by-reach", "two-rounds-d64", "two-rounds-d128", "shared",
+        "shared-three", "own-order", "own-order-d256",
         "two", "two-histories"])
 def test_tile_orders_by_rounds(q_lens, step, heads, dim):
     """Each order, at one workgroup a CU (D = 128, 256) and two (D = 64)."""

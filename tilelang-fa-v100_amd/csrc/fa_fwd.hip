@@ -337,12 +337,13 @@ struct PagedOrder {
 // history in units of a tile's rows, u_b + i + 1 the reach of tile i:
 //  * by sequence, each from its longest tile: grids of no more workgroups (tiles x
 //    combos) than CUs, a single sequence or two short prompts (the search below
-//    costs 0.5-1 us a workgroup), and more than two rounds without histories to
-//    tell sequences apart;
-//  * up to two rounds: all tiles by decreasing reach, ties by sequence.
+//    costs 0.5-1 us a workgroup), and more rounds than the next item's without
+//    histories to tell sequences apart;
+//  * up to two rounds (kPagedTileOrderRounds; three where XCDs share combos): all
+//    tiles by decreasing reach, ties by sequence.
 //    Sequence b has n_b(K) = clamp(u_b + ntiles_b - K, 0, ntiles_b) tiles of
 //    reach above K;
-//  * more than two rounds: sequences by the reach of their last tile, longest
+//  * more rounds: sequences by the reach of their last tile, longest
 //    first (the tiles of one share its K / V in the L2), n_b(K) = all or none.
 // For the last two a search for the smallest K with at most `tile` tiles above
 // it, and the slot's rank among those at K, name the tile.  More sequences are
@@ -364,7 +365,9 @@ __device__ int find_sequence(const int32_t* qsl, const int32_t* prefix, int batc
       const int total = __builtin_amdgcn_readlane(last, 63);
       const int64_t wgs = (int64_t)total * combos;
       int here = n, before = 0, rank = tile;
-      const bool by_tile = wgs <= 2 * (int64_t)order.one_round;
+      const int rounds = combos % kOrderXcds == 0 ? tiles::kPagedTileOrderRounds
+                                                  : tiles::kPagedTileOrderRoundsShared;
+      const bool by_tile = wgs <= rounds * (int64_t)order.one_round;
       const uint64_t some = __ballot(n > 0);
       if (wgs > order.cus && tile < total && __popcll(some) > 1) {
         const int u0 = __builtin_amdgcn_readlane(u, __ffsll((unsigned long long)some) - 1);

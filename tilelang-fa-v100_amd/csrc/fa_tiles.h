@@ -226,8 +226,10 @@ constexpr int kMaxSplits = 64;
 constexpr int64_t kSplitByRangeTokens = 512;
 
 // ---- workgroup order of the paged kernels (fa_fwd.hip paged_order,
-// find_sequence).  Up to two rounds of (tile, KV head, key range) workgroups
-// (CUs x workgroups per CU is one) every tile goes by its own reach; above, whole
+// find_sequence).  Up to kPagedTileOrderRounds rounds of (tile, KV head, key range)
+// workgroups (CUs x workgroups per CU is one) every tile goes by its own reach, up
+// to kPagedTileOrderRoundsShared where (KV head, key range) pairs are no multiple
+// of the 8 XCDs, which then share them and their K / V anyway; above, whole
 // sequences by their reach where histories differ, else in their own order.
 // Evidence (us, same box, D = 128 unless noted, against combo-major ranges of ids
 // with sequences by history): 8 prompts of 512-4096 tokens, 16 / 2 heads 281 -> 262;
@@ -236,7 +238,12 @@ constexpr int64_t kSplitByRangeTokens = 512;
 // chunks + 30 one-token sequences, 2 ranges 158 -> 150.  The tile order loses the
 // K / V reuse in the L2, so it stops at two rounds: 27 prompts of 356-712 tokens,
 // 32 / 8 heads (1900 workgroups) 140 by sequence, 153 by tile; 8 of 512-4096 (2400)
-// 467 and 474.
+// 467 and 474.  Between two and 3.3 rounds, over 69 drawn batches with 2 or 4 KV heads
+// the tile order up to three rounds is 2.5% faster than up to two (three prompts of
+// 1491-1884 tokens, 28 / 4 90.4 -> 87.0, where combo-major took 84; 23 of 313-626, 16 / 2
+// 57.7 -> 49.8; the most it loses is 8%, four chunks of 614-1228 among 25 one-token
+// sequences, 28 / 4).  Over 70 with 8 or 16 it gains nothing and costs up to 19% (four of
+// 183-366, 64 / 8, D = 256 37.9 by sequence, 45.2 by tile).
 // The search for a workgroup's tile takes 0.5-1 us, so a single sequence and two
 // prompts below kPagedOrderPairKeys go without it (searched / by sequence: one of
 // 535-1070 tokens, 64 / 8 heads, D = 256 47.3 / 45.4; two of 434-868, 64 / 8 37.4 /
@@ -246,6 +253,8 @@ constexpr int64_t kSplitByRangeTokens = 512;
 // 117 / 144).  Two rounds are 1024 workgroups at D = 64, which runs two a CU (14 of
 // 185-370, 28 / 4 27.1 by tile, 29.0 by sequence; 4 of 736-1472, 16 / 16 33.9, 40.4).
 constexpr int kPagedOrderPairKeys = 1024;
+constexpr int kPagedTileOrderRounds = 2;
+constexpr int kPagedTileOrderRoundsShared = 3;
 
 // ---- paged tiles of at most 32 rows (fa_fwd.hip run_paged_tile, paged_few_rows):
 // their keys are split over the workgroup's waves from kPagedFewMinKeys keys (of
