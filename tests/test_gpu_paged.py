@@ -101,6 +101,15 @@ def test_sliding_windows(D):
         check(c, causal=True, wq=wq, wk=wk)
 
 
+@pytest.mark.parametrize("D", [64, 128, 256, 512])
+def test_windows_at_the_end_of_32_bits(D):
+    """2^31 - 1, as "unbounded" is often written, and 100 less; few rows, many rows and split."""
+    big = 2 ** 31 - 1
+    c = make_case(8, [200, 77, 2, 0], [500, 77, 4200, 9], [300, 0, 4198, 9], 8, 4, D)
+    for wq, wk in ((big, big), (-1, big - 100), (64, big), (big, 33)):
+        check(c, causal=True, wq=wq, wk=wk)
+
+
 @pytest.mark.parametrize("page,D", [(32, 64), (1, 128), (32, 128), (128, 128), (64, 256), (16, 512)])
 def test_page_sizes_and_head_dims(page, D):
     c = make_case(5, [150, 260], [400, 260], [250, 0], 4, 2, D, page=page)

@@ -471,7 +471,9 @@ __device__ __forceinline__ void paged_rows(const Args& a, int hk, int b, int qs,
   P.prefix = a.prefix_kv_lens[b];
   P.causal = a.causal != 0;
   P.wq = a.window_q;
-  P.wk = a.window_k;
+  // (A bound of the sequence's length hides nothing; with one near 2^31, token
+  // + bound would leave 32 bits.)
+  P.wk = min(a.window_k, P.seq_len);
 }
 
 // One row tile of a paged problem, which sees up to keys() keys; setup(args, P)
